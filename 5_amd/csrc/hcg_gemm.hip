@@ -21,6 +21,9 @@
 //     cleared in the last K tile), and an LDS-staged 16-byte epilogue;
 //     shapes with few tiles and a long K split K over workgroups (partials
 //     summed in a fixed order by stream_reduce_kernel).
+//   * wg8::gemm_wg8_kernel (hcg_wg8.h) -- eight waves per workgroup on
+//     128x128, 64x64, 64x128 or 128x256 tiles: shapes whose 256-row tiles
+//     would leave most CUs idle.
 //   * gemm_stream_kernel -- M <= 128, N > 64 (HBM-bound).  B streams HBM ->
 //     LDS once by DMA, split over K across workgroups mapped so every XCD
 //     covers all column residues, against 1, 2, 4 or 8 16-row blocks of A;
@@ -427,6 +430,12 @@ struct WgStamps {
   __device__ __forceinline__ void write() {}
 #endif
 };
+
+}  // namespace
+
+#include "hcg_wg8.h"
+
+namespace {
 
 template <int TM>
 constexpr int dma_stage_bytes() {
@@ -2429,70 +2438,83 @@ int launch_generic(const TiledArgs& a, bool vec_a, bool vec_b, hipStream_t strea
   return HCG_OK;
 }
 
-// Output tile shapes of the DMA kernel.  TM = 256: 4-stage ring, one
-// workgroup per CU; TM = 128: 3-stage ring, two workgroups per CU.
+// Output tile shapes: those of gemm_dma_kernel (K step 32; TM = 256: 4-stage
+// ring, one workgroup per CU; TM = 128: 3-stage ring, two per CU) and those
+// of wg8::gemm_wg8_kernel (K step 64).  The first five are HCG_ALGO_TILED_*
+// in order.
+//
+// Modelled time, us: kLaunchUs + rounds * fixed + (tiles of the busiest CU) *
+// (K steps) * step, where a round is per_cu workgroups resident on a CU.
+// The constants are a least-squares fit (of log time) to 110 shapes, M, N
+// and K log-uniform in 65..8192, bf16, every tile shape timed on each and
+// the wg8 shapes with 1, 2, 4 and 8 K splits: the pick was within 0.3% of
+// the fastest shape on average and at most 8% off (7172 x 1856 x 704).
+// What the wg8 shapes changed (us, the fastest gemm_dma_kernel shape ->
+// wg8): 256^3 5.2 -> 3.7 (64x64), 1000^3 14.4 -> 7.8 (64x64),
+// 8192 x 128 x 2048 21.0 -> 8.8 (64x64), 512 x 4096 x 4096 37.9 -> 22.4
+// (64x128), 2048^3 23.2 -> 18.2 (128x128), 2500^3 38.7 -> 35.7 (128x256);
+// 128 x 128 tiles of gemm_dma_kernel were never the fastest and are gone,
+// its 256-row tiles stay ahead from about 256 of them (3000^3 54.4 against
+// 78.2) and its 128x256 tiles, two workgroups per CU, where a CU takes two
+// or more (8192 x 8192 x 256 60.5 against 70.5).
 struct TileShape {
   int tm, tn;
-  int per_cu;   // workgroups resident per CU
-  float eff;    // relative MFMA issue efficiency of the K loop (measured)
+  int per_cu;  // workgroups resident per CU
+  int ks;      // K step
+  bool wg8;
+  float fixed, step;
 };
 constexpr TileShape kTileShapes[] = {
-    {256, 256, 1, 1.00f},
-    {256, 192, 1, 0.97f},
-    {128, 256, 2, 0.93f},
-    {128, 128, 2, 0.75f},
-    {256, 64, 1, 0.75f},  // narrow N (<= 64): the A stream dominates
+    {256, 256, 1, 32, false, 8.13f, 0.487f},
+    {256, 192, 1, 32, false, 7.89f, 0.409f},
+    {128, 256, 2, 32, false, 3.75f, 0.350f},
+    {128, 128, 1, 64, true, 3.27f, 0.434f},
+    {256, 64, 1, 32, false, 7.0f, 0.20f},  // (forced only: narrow N is the narrow kernel's, or 64x64 tiles')
+    {64, 64, 2, 64, true, 1.73f, 0.218f},
+    {64, 128, 1, 64, true, 2.20f, 0.312f},
+    {128, 256, 1, 64, true, 4.74f, 0.610f},
 };
 constexpr int kNumTileShapes = sizeof(kTileShapes) / sizeof(kTileShapes[0]);
+constexpr int kNarrowShape = 4;
+constexpr double kLaunchUs = 1.9;
 
-// Picks the tile shape with the least modelled time: the busiest CU's
-// share of tiles times tile area times K steps (scaled by the shape's K-loop
-// efficiency), plus a fixed cost per round of resident workgroups
-// (prologue, epilogue, launch) worth about eight 256x256 K tiles, or four
-// where two workgroups share a CU and each hides part of the other's.  The
-// constants were fitted to 24 shapes timed with every tile shape forced;
-// the pick was within 6% of the fastest on all of them.
+// Picks the tile shape with the least modelled time.
 //
 // With splits > 1 (split-K), each tile's K range is cut into `splits`
 // parts run by separate workgroups whose partial products a second kernel
 // sums in a fixed order; that reduction is charged as its launch plus the
-// partials' HBM traffic ((splits + 1) x M x N floats), converted to K tiles
-// at 0.73 us per 256x256 K tile.
+// partials' HBM traffic ((splits + 1) x M x N floats).
 struct TilePlan {
   int shape;
   int splits;
 };
 
-constexpr int kSplitCandidates[] = {1, 2, 3, 4, 6, 8};
-constexpr int kMinKTilesPerSplit = 8;
+constexpr int kSplitCandidates[] = {1, 2, 3, 4, 6, 8, 12, 16};
+constexpr int kMinKPerSplit = 256;
 constexpr size_t kMaxSplitWorkspace = (size_t)512 << 20;
 
 // `room`: scratch bytes available for the partials (kMaxSplitWorkspace at
 // most).
 bool split_ok(int splits, int M, int N, int K, size_t room) {
-  const int nk = (K + kDmaK - 1) / kDmaK;
   const size_t limit = room < kMaxSplitWorkspace ? room : kMaxSplitWorkspace;
-  return splits == 1 || (splits <= 64 && (nk + splits - 1) / splits >= kMinKTilesPerSplit &&
+  return splits == 1 || (splits <= 64 && (K + splits - 1) / splits >= kMinKPerSplit &&
                          (size_t)splits * M * N * sizeof(float) <= limit);
 }
 
+// Microseconds (see TileShape).
 double plan_cost(const TileShape& t, int splits, int num_cus, int M, int N, int K) {
-  const int64_t nk = (K + kDmaK - 1) / kDmaK;
+  const int64_t nk = ((K + t.ks - 1) / t.ks + splits - 1) / splits;
   const int64_t tiles = (int64_t)((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn) * splits;
   const int64_t per_cu = (tiles + num_cus - 1) / num_cus;
   const int64_t rounds = (per_cu + t.per_cu - 1) / t.per_cu;
-  const double fixed = t.per_cu == 1 ? 8.0 : 4.0;
-  const double unit = 256.0 * 256.0;
-  double cost = (double)per_cu * t.tm * t.tn * (double)((nk + splits - 1) / splits) / t.eff + (double)rounds * fixed * unit;
-  if (splits > 1) {
-    const double reduce_us = 2.0 + (double)(splits + 1) * M * N * sizeof(float) / 4.5e6;
-    cost += reduce_us / 0.73 * unit;
-  }
-  return cost;
+  double us = kLaunchUs + (double)rounds * t.fixed + (double)(per_cu * nk) * t.step;
+  if (splits > 1) us += 2.0 + (double)(splits + 1) * M * N * sizeof(float) / 4.5e6;
+  return us;
 }
 
+// wide: operands that need gemm_dma_kernel's WIDE form (no wg8 shape has one).
 TilePlan plan_tiles(int num_cus, int M, int N, int K, int force_shape, bool allow_split,
-                    double* cost_out = nullptr, size_t room = kMaxSplitWorkspace) {
+                    double* cost_out = nullptr, size_t room = kMaxSplitWorkspace, bool wide = false) {
   TilePlan best{force_shape >= 0 ? force_shape : 0, 1};
   double best_cost = -1;
   const int forced_splits =
@@ -2500,8 +2522,9 @@ TilePlan plan_tiles(int num_cus, int M, int N, int K, int force_shape, bool allo
           ? g_tiled_splits_override
           : 0;
   for (int i = 0; i < kNumTileShapes; ++i) {
-    if (force_shape >= 0 && i != force_shape) continue;
     const TileShape& t = kTileShapes[i];
+    if (force_shape >= 0 ? i != force_shape : i == kNarrowShape && N > 64) continue;
+    if (wide && force_shape < 0 && t.wg8) continue;
     if ((int64_t)((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn) * 64 > 0x7fffffff) continue;
     for (int c = 0; c < (forced_splits > 0 ? 1 : (int)(sizeof(kSplitCandidates) / sizeof(int))); ++c) {
       const int splits = forced_splits > 0 ? forced_splits : kSplitCandidates[c];
@@ -2519,8 +2542,46 @@ TilePlan plan_tiles(int num_cus, int M, int N, int K, int force_shape, bool allo
 }
 
 
+template <int DT, bool KT>
+int launch_wg8(const FastArgs& f, int shape, hipStream_t stream) {
+  hcg::wg8::Args a{};
+  a.A = f.A;
+  a.B = f.B;
+  a.C = f.C;
+  a.lda = f.lda;
+  a.ldb = f.ldb;
+  a.ldc = f.ldc;
+  a.M = f.M;
+  a.N = f.N;
+  a.K = f.K;
+  a.tiles_m = f.tiles_m;
+  a.tiles_n = f.tiles_n;
+  a.a_bytes = f.a_bytes;
+  a.b_bytes = f.b_bytes;
+  a.c_vec = f.c_vec;
+  a.splits = f.splits;
+  a.kchunk = f.kchunk;
+  a.ws = f.ws;
+  a.ws_vec = f.ws_vec;
+  const dim3 grid((unsigned)(a.tiles_m * a.tiles_n * a.splits));
+  const dim3 block(hcg::wg8::kThreads);
+  HCG_STAMP_ARGS(hcg::wg8::Args, a)
+  using namespace hcg::wg8;
+  switch (shape) {
+    case 3: gemm_wg8_kernel<DT, 128, 128, 2, 2, 64, 4, true, false, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
+    case 5: gemm_wg8_kernel<DT, 64, 64, 2, 2, 64, 4, true, false, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
+    case 6: gemm_wg8_kernel<DT, 64, 128, 2, 2, 64, 4, true, false, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
+    default: gemm_wg8_kernel<DT, 128, 256, 2, 4, 64, 3, true, false, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
+  }
+  HCG_HIP_CHECK(hipGetLastError());
+  return HCG_OK;
+}
+
 template <int DT, bool WIDE, bool KT = false>
 int launch_dma(const FastArgs& a, int shape, hipStream_t stream) {
+  if constexpr (!WIDE) {
+    if (kTileShapes[shape].wg8) return launch_wg8<DT, KT>(a, shape, stream);
+  }
   const dim3 grid((unsigned)(a.tiles_m * a.tiles_n * (a.splits > 1 ? a.splits : 1)));
   const dim3 block(kTiledThreads);
   HCG_STAMP_ARGS(FastArgs, a)
@@ -2530,9 +2591,11 @@ int launch_dma(const FastArgs& a, int shape, hipStream_t stream) {
   switch (shape) {
     case 0: gemm_dma_kernel<DT, 256, 256, 4, WIDE, KT, kA2><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
     case 1: gemm_dma_kernel<DT, 256, 192, 4, WIDE, KT, kA2><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
-    case 2: gemm_dma_kernel<DT, 128, 256, 3, WIDE, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
-    case 3: gemm_dma_kernel<DT, 128, 128, 3, WIDE, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
-    default: gemm_dma_kernel<DT, 256, 64, 4, WIDE, KT, kA2><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
+    case 3:  // (WIDE only: 128x128 tiles otherwise run on wg8)
+      if constexpr (WIDE) gemm_dma_kernel<DT, 128, 128, 3, WIDE, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a));
+      break;
+    case 4: gemm_dma_kernel<DT, 256, 64, 4, WIDE, KT, kA2><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
+    default: gemm_dma_kernel<DT, 128, 256, 3, WIDE, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
   }
   HCG_HIP_CHECK(hipGetLastError());
   return HCG_OK;
@@ -2935,7 +2998,7 @@ int run_tiled(const Scratch& sc, int dtype, const void* A, int64_t lda, const vo
                     (int64_t)kDmaK * ldb * 2 < kLimit && tiles <= 0x7fffffff;
   if (force_generic || (!fits && !wide)) return run_generic(dtype, A, lda, B, ldb, C, ldc, M, N, K, stream);
   if (wide) {
-    const TilePlan plan = plan_tiles(st->num_cus, M, N, K, force_shape, false);
+    const TilePlan plan = plan_tiles(st->num_cus, M, N, K, force_shape, false, nullptr, 0, true);
     const TileShape& ts = kTileShapes[plan.shape];
     FastArgs f{};
     f.A = static_cast<const uint16_t*>(A);
@@ -3009,9 +3072,9 @@ int run_tiled(const Scratch& sc, int dtype, const void* A, int64_t lda, const vo
   f.c_vec = aligned16(C) && ldc % 4 == 0;
   f.splits = 1;
   if (plan.splits > 1) {
-    // K cut into equal runs of whole 32-row K tiles; no split is empty.
-    const int nk = (K + kDmaK - 1) / kDmaK;
-    f.kchunk = (nk + plan.splits - 1) / plan.splits * kDmaK;
+    // K cut into equal runs of whole K steps; no split is empty.
+    const int nk = (K + ts.ks - 1) / ts.ks;
+    f.kchunk = (nk + plan.splits - 1) / plan.splits * ts.ks;
     f.splits = (K + f.kchunk - 1) / f.kchunk;
     f.ws = reinterpret_cast<float*>(static_cast<char*>(ws) + a_sz + b_sz);
     f.ws_vec = N % 4 == 0;  // 16-byte partial rows (the workspace base is 256-byte aligned)
@@ -3040,11 +3103,10 @@ double tiled_cost(int num_cus, int M, int N, int K) {
   return cost;
 }
 
-// A streaming launch in the tile model's units (0.73 us per 256 x 256 x 1):
-// a fixed 8 us (launch behind the tiled kernel, ramp-up, the K split's
-// reduce) plus its bytes at 5 TB/s.  Fitted so that short-K shapes
+// A streaming launch in microseconds: a fixed 8 us (launch behind the tiled
+// kernel, ramp-up, the K split's reduce) plus its bytes at 5 TB/s.  Fitted so that short-K shapes
 // (4100 x 4096 x 256: 20.4 us unpeeled, 23.1 us peeled) stay unpeeled.
-double stream_units(double bytes) { return (8.0 + bytes / 5.0e6) / 0.73 * 65536.0; }
+double stream_us(double bytes) { return 8.0 + bytes / 5.0e6; }
 
 Peel plan_peel(const DeviceState* st, const void* A, int64_t lda, const void* B, int64_t ldb, int M, int N,
                int K) {
@@ -3054,7 +3116,7 @@ Peel plan_peel(const DeviceState* st, const void* A, int64_t lda, const void* B,
   if (M > 256 && rm > 0 && rm <= 128 &&
       (rm <= 16 || stream_fits(static_cast<const uint16_t*>(A) + (int64_t)(M - rm) * lda, lda, B, ldb, rm, N, K))) {
     const double c = tiled_cost(st->num_cus, M - rm, N, K) +
-                     stream_units(2.0 * K * N + 2.0 * rm * K + 4.0 * rm * N);
+                     stream_us(2.0 * K * N + 2.0 * rm * K + 4.0 * rm * N);
     if (c < best) {
       best = c;
       p.rows = rm;
@@ -3064,7 +3126,7 @@ Peel plan_peel(const DeviceState* st, const void* A, int64_t lda, const void* B,
   if (N > 256 && rn > 0 && rn <= 64 &&
       rowstream_fits(A, lda, static_cast<const uint16_t*>(B) + (N - rn), ldb, M, rn, K)) {
     const double c = tiled_cost(st->num_cus, M, N - rn, K) +
-                     stream_units(2.0 * M * K + 2.0 * K * rn + 4.0 * M * rn);
+                     stream_us(2.0 * M * K + 2.0 * K * rn + 4.0 * M * rn);
     if (c < best) {
       best = c;
       p.rows = 0;

@@ -1,0 +1,78 @@
+"""The eight-wave tiled kernel (5_amd/csrc/hcg_wg8.h) at the edges of its tiles.
+
+Small-integer operands make every sum exact in float32 whatever its order, so
+C must equal A @ B bit for bit.  A and B are views into NaN-filled buffers
+(NaN past K in A's rows and past N in B's: no element outside a view may reach
+C) and C is a view into a NaN-filled buffer whose other elements must stay.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+DEV = "cuda:0"
+DTYPES = {"float16": torch.float16, "bfloat16": torch.bfloat16}
+
+
+def _padded(x, dtype, pad):
+    rows, cols = x.shape
+    buf = torch.full((rows + 1, cols + pad), float("nan"), dtype=dtype, device=DEV)
+    buf[:rows, :cols] = torch.from_numpy(x.astype(np.float32)).to(DEV).to(dtype)
+    return buf[:rows, :cols]
+
+
+def _check(m, n, k, dtype, pad, algo="auto"):
+    import hc.gfx950 as g
+
+    print(f"case wg8 {dtype} m={m} n={n} k={k} pad={pad} algo={algo}", flush=True)
+    rng = np.random.default_rng(m + 3 * n + 7 * k)
+    ai, bi = rng.integers(-4, 5, size=(m, k)), rng.integers(-4, 5, size=(k, n))
+    a, b = _padded(ai, DTYPES[dtype], pad), _padded(bi, DTYPES[dtype], pad)
+    guard = torch.full((m + 2, n + pad), float("nan"), dtype=torch.float32, device=DEV)
+    for _ in range(2):  # the second call reuses the stream's workspace
+        g.gemm(a, b, out=guard[:m, :n], algo=algo)
+    torch.cuda.synchronize()
+    got = guard.cpu().numpy()
+    assert np.array_equal(got[:m, :n], (ai.astype(np.float64) @ bi.astype(np.float64)).astype(np.float32))
+    assert np.all(np.isnan(got[m:])) and np.all(np.isnan(got[:, n:]))
+
+
+# Tiles of 64x64 (one and two a side, K below, at and past one and several
+# 64-wide steps), 64x128, 128x128 and 128x256, each with ragged and whole
+# edges, as the plan picks them for these sizes.
+_SHAPES = [
+    (65, 65, 1), (65, 66, 63), (127, 129, 64), (129, 190, 257), (128, 128, 128), (500, 1000, 512),
+    (200, 8192, 1000), (170, 6019, 264),
+    (1664, 2000, 200), (1601, 2041, 264), (2048, 2048, 520),
+    (2500, 2500, 1000), (576, 7232, 768), (8192, 1024, 1024),
+]
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("m,n,k", _SHAPES)
+def test_wg8_tiles(m, n, k, dtype):
+    _check(m, n, k, dtype, 8)
+
+
+@pytest.mark.parametrize("pad", [0, 1, 4, 5])
+@pytest.mark.parametrize("m,n,k", [(129, 190, 261), (170, 6019, 70), (1601, 2041, 65)])
+def test_wg8_row_alignment(m, n, k, pad):
+    """Rows of A, B and C at every alignment class (K and N odd or not)."""
+    _check(m, n, k, "float16", pad)
+
+
+@pytest.mark.parametrize("m,n,k", [(512, 512, 16384), (130, 200, 8200), (128, 8192, 8192), (333, 444, 4999),
+                                   (192, 136, 1536)])
+def test_wg8_split_k(m, n, k):
+    _check(m, n, k, "bfloat16", 4)
+    _check(m, n, k, "float16", 3)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (128, 128, 31), (129, 257, 96), (640, 384, 1000)])
+def test_forced_128x128(m, n, k):
+    _check(m, n, k, "float16", 4, "tiled_128x128")
