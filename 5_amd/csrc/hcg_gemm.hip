@@ -317,6 +317,8 @@ struct FastArgs {
   int splits, kchunk;
   float* ws;
   bool ws_vec;           // N is a multiple of 4 (16-byte partial rows)
+  unsigned* counters;    // wg8 only: arrival counters of the fused reduction, or null
+  int ws_bytes;          // (with counters) bytes of the partials, below 2^31
 #ifdef HCG_STAMPS
   int stamp_slot;
 #endif
@@ -2443,12 +2445,15 @@ int launch_generic(const TiledArgs& a, bool vec_a, bool vec_b, hipStream_t strea
 // of wg8::gemm_wg8_kernel (K step 64).  The first five are HCG_ALGO_TILED_*
 // in order.
 //
-// Modelled time, us: kLaunchUs + rounds * fixed + (tiles of the busiest CU) *
-// (K steps) * step, where a round is per_cu workgroups resident on a CU.
-// The constants are a least-squares fit (of log time) to 110 shapes, M, N
-// and K log-uniform in 65..8192, bf16, every tile shape timed on each and
-// the wg8 shapes with 1, 2, 4 and 8 K splits: the pick was within 0.3% of
-// the fastest shape on average and at most 8% off (7172 x 1856 x 704).
+// Modelled time, us: kLaunchUs + rounds * fixed + (units of the busiest CU) *
+// (K steps) * step, where a unit is one K split of one tile, a round is
+// per_cu units resident on a CU, and step goes from lo (one busy CU) to hi
+// (all busy: shared bandwidth, lower clock).  The constants are a
+// least-squares fit (of log time) to 214 shapes (M, N and K log-uniform in
+// 65..8192, few rows or columns over K up to 32768, up to 64 rows), bf16,
+// every tile shape timed on each, the wg8 shapes with up to 16 K splits: the
+// pick was within 0.7% of the fastest on average over the first kind and
+// 2.6% over the others.
 // What the wg8 shapes changed (us, the fastest gemm_dma_kernel shape ->
 // wg8): 256^3 5.2 -> 3.7 (64x64), 1000^3 14.4 -> 7.8 (64x64),
 // 8192 x 128 x 2048 21.0 -> 8.8 (64x64), 512 x 4096 x 4096 37.9 -> 22.4
@@ -2462,35 +2467,44 @@ struct TileShape {
   int per_cu;  // workgroups resident per CU
   int ks;      // K step
   bool wg8;
-  float fixed, step;
+  float fixed, lo, hi;
 };
 constexpr TileShape kTileShapes[] = {
-    {256, 256, 1, 32, false, 8.13f, 0.487f},
-    {256, 192, 1, 32, false, 7.89f, 0.409f},
-    {128, 256, 2, 32, false, 3.75f, 0.350f},
-    {128, 128, 1, 64, true, 3.27f, 0.434f},
-    {256, 64, 1, 32, false, 7.0f, 0.20f},  // (forced only: narrow N is the narrow kernel's, or 64x64 tiles')
-    {64, 64, 2, 64, true, 1.73f, 0.218f},
-    {64, 128, 1, 64, true, 2.20f, 0.312f},
-    {128, 256, 1, 64, true, 4.74f, 0.610f},
+    {256, 256, 1, 32, false, 8.04f, 0.443f, 0.674f},
+    {256, 192, 1, 32, false, 7.81f, 0.377f, 0.501f},
+    {128, 256, 2, 32, false, 3.78f, 0.303f, 0.419f},
+    {128, 128, 1, 64, true, 3.07f, 0.352f, 0.523f},
+    {256, 64, 1, 32, false, 7.0f, 0.20f, 0.25f},  // (N <= 64 only)
+    {64, 64, 2, 64, true, 1.26f, 0.183f, 0.261f},
+    {64, 128, 1, 64, true, 1.89f, 0.263f, 0.366f},
+    {128, 256, 1, 64, true, 4.32f, 0.484f, 0.828f},
 };
 constexpr int kNumTileShapes = sizeof(kTileShapes) / sizeof(kTileShapes[0]);
 constexpr int kNarrowShape = 4;
-constexpr double kLaunchUs = 1.9;
+constexpr double kLaunchUs = 2.0;
 
-// Picks the tile shape with the least modelled time.
+// Picks the tile shape and K split with the least modelled time.
 //
-// With splits > 1 (split-K), each tile's K range is cut into `splits`
-// parts run by separate workgroups whose partial products a second kernel
-// sums in a fixed order; that reduction is charged as its launch plus the
-// partials' HBM traffic ((splits + 1) x M x N floats).
+// With splits > 1 (split-K), each tile's K range is cut into `splits` parts
+// run by separate workgroups, whose partial products are summed in the order
+// of the parts, bit-reproducibly: by the tile's last workgroup to arrive
+// (fused: wg8 tiles of at most 128x128), or by a second launch.  Fused, the
+// tail of a workgroup grows by 1 us (write-through, atomic) plus the other
+// partials' loads at 100 KB/us by one CU, plus the partials' traffic; the
+// second launch costs 3 to 6 us (boxes differ by the gap between launches)
+// plus the traffic, and 2.5 us of host time, so that small calls take at
+// least 6.6 us.  Both sides, us: 128 x 8192 x 8192 (4 parts of 64 KB) 34.4
+// fused, 35.8 not; 1024 x 1024 x 4096 14.7 / 16.3; 192 x 192 x 1440 5.7 /
+// 6.8; 512 x 512 x 16384 in 16 parts 26.4 / 15.8.
 struct TilePlan {
   int shape;
   int splits;
+  bool fused;
 };
 
 constexpr int kSplitCandidates[] = {1, 2, 3, 4, 6, 8, 12, 16};
 constexpr int kMinKPerSplit = 256;
+constexpr int kMinKPerFusedSplit = 128;
 constexpr size_t kMaxSplitWorkspace = (size_t)512 << 20;
 
 // `room`: scratch bytes available for the partials (kMaxSplitWorkspace at
@@ -2501,21 +2515,45 @@ bool split_ok(int splits, int M, int N, int K, size_t room) {
                          (size_t)splits * M * N * sizeof(float) <= limit);
 }
 
-// Microseconds (see TileShape).
-double plan_cost(const TileShape& t, int splits, int num_cus, int M, int N, int K) {
+int64_t plan_tile_count(const TileShape& t, int M, int N) {
+  return (int64_t)((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn);
+}
+// Bytes of the fused reduction's partials (whole tiles).
+size_t fused_bytes(const TileShape& t, int splits, int M, int N) {
+  return (size_t)splits * (size_t)plan_tile_count(t, M, N) * t.tm * t.tn * sizeof(float);
+}
+bool fused_ok(const TileShape& t, int splits, int M, int N, int K, size_t room) {
+  const size_t limit = room < kMaxSplitWorkspace ? room : kMaxSplitWorkspace;
+  return t.wg8 && hcg::wg8::can_fuse(t.tm, t.tn) && splits > 1 && splits <= 16 &&
+         (K + splits - 1) / splits >= kMinKPerFusedSplit &&
+         plan_tile_count(t, M, N) * hcg::wg8::kCounterStride * 4 <= kStCounterBytes &&
+         fused_bytes(t, splits, M, N) <= limit;
+}
+
+// Microseconds (see TileShape and TilePlan).
+double plan_cost(const TileShape& t, int splits, bool fused, int num_cus, int M, int N, int K) {
   const int64_t nk = ((K + t.ks - 1) / t.ks + splits - 1) / splits;
-  const int64_t tiles = (int64_t)((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn) * splits;
-  const int64_t per_cu = (tiles + num_cus - 1) / num_cus;
+  const int64_t units = plan_tile_count(t, M, N) * splits;
+  const int64_t per_cu = (units + num_cus - 1) / num_cus;
   const int64_t rounds = (per_cu + t.per_cu - 1) / t.per_cu;
-  double us = kLaunchUs + (double)rounds * t.fixed + (double)(per_cu * nk) * t.step;
-  if (splits > 1) us += 2.0 + (double)(splits + 1) * M * N * sizeof(float) / 4.5e6;
+  const double busy = units < num_cus ? (double)units / num_cus : 1.0;
+  double us = kLaunchUs + (double)rounds * t.fixed + (double)(per_cu * nk) * (t.lo + (t.hi - t.lo) * busy);
+  if (splits > 1) {
+    if (fused) {
+      us += 1.0 + (splits - 1) * (t.tm * t.tn * 4) / 1.0e5 + (double)fused_bytes(t, splits, M, N) / 3.0e6;
+    } else {
+      us += 4.2 + (double)(splits + 1) * M * N * sizeof(float) / 4.5e6;
+      if (us < 6.6) us = 6.6;
+    }
+  }
   return us;
 }
 
-// wide: operands that need gemm_dma_kernel's WIDE form (no wg8 shape has one).
-TilePlan plan_tiles(int num_cus, int M, int N, int K, int force_shape, bool allow_split,
-                    double* cost_out = nullptr, size_t room = kMaxSplitWorkspace, bool wide = false) {
-  TilePlan best{force_shape >= 0 ? force_shape : 0, 1};
+// wide: operands that need gemm_dma_kernel's WIDE form (no wg8 shape has
+// one).  fuse: the caller's scratch has arrival counters.
+TilePlan plan_tiles(int num_cus, int M, int N, int K, int force_shape, bool allow_split, double* cost_out = nullptr,
+                    size_t room = kMaxSplitWorkspace, bool wide = false, bool fuse = true) {
+  TilePlan best{force_shape >= 0 ? force_shape : 0, 1, false};
   double best_cost = -1;
   const int forced_splits =
       allow_split && g_tiled_splits_override > 0 && split_ok(g_tiled_splits_override, M, N, K, room)
@@ -2525,22 +2563,23 @@ TilePlan plan_tiles(int num_cus, int M, int N, int K, int force_shape, bool allo
     const TileShape& t = kTileShapes[i];
     if (force_shape >= 0 ? i != force_shape : i == kNarrowShape && N > 64) continue;
     if (wide && force_shape < 0 && t.wg8) continue;
-    if ((int64_t)((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn) * 64 > 0x7fffffff) continue;
+    if (plan_tile_count(t, M, N) * 64 > 0x7fffffff) continue;
     for (int c = 0; c < (forced_splits > 0 ? 1 : (int)(sizeof(kSplitCandidates) / sizeof(int))); ++c) {
       const int splits = forced_splits > 0 ? forced_splits : kSplitCandidates[c];
       if (splits > 1 && !allow_split) break;
-      if (!split_ok(splits, M, N, K, room)) continue;
-      const double cost = plan_cost(t, splits, num_cus, M, N, K);
-      if (best_cost < 0 || cost < best_cost) {
-        best = TilePlan{i, splits};
-        best_cost = cost;
+      for (int f = 0; f < 2; ++f) {
+        if (f ? !(fuse && fused_ok(t, splits, M, N, K, room)) : !split_ok(splits, M, N, K, room)) continue;
+        const double cost = plan_cost(t, splits, f != 0, num_cus, M, N, K);
+        if (best_cost < 0 || cost < best_cost) {
+          best = TilePlan{i, splits, f != 0};
+          best_cost = cost;
+        }
       }
     }
   }
   if (cost_out) *cost_out = best_cost;
   return best;
 }
-
 
 template <int DT, bool KT>
 int launch_wg8(const FastArgs& f, int shape, hipStream_t stream) {
@@ -2563,6 +2602,8 @@ int launch_wg8(const FastArgs& f, int shape, hipStream_t stream) {
   a.kchunk = f.kchunk;
   a.ws = f.ws;
   a.ws_vec = f.ws_vec;
+  a.counters = f.counters;
+  a.ws_bytes = f.ws_bytes;
   const dim3 grid((unsigned)(a.tiles_m * a.tiles_n * a.splits));
   const dim3 block(hcg::wg8::kThreads);
   HCG_STAMP_ARGS(hcg::wg8::Args, a)
@@ -3023,14 +3064,17 @@ int run_tiled(const Scratch& sc, int dtype, const void* A, int64_t lda, const vo
   const size_t b_sz = b_ok ? 0 : round_up((size_t)K * ldb_p * 2, 256);
   // Explicit tile shapes run without a K split; "auto" and "tiled" may split.
   const TilePlan plan = plan_tiles(st->num_cus, M, N, K, force_shape, force_shape < 0, nullptr,
-                                   sc.room(a_sz + b_sz));
+                                   sc.room(a_sz + b_sz), false, sc.fixed == nullptr);
   const TileShape& ts = kTileShapes[plan.shape];
   if ((int64_t)((M + ts.tm - 1) / ts.tm) * ((N + ts.tn - 1) / ts.tn) * plan.splits > 0x7fffffff)
     return run_generic(dtype, A, lda, B, ldb, C, ldc, M, N, K, stream);
-  const size_t p_sz = plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0;
+  const size_t p_sz = plan.fused        ? fused_bytes(ts, plan.splits, M, N)
+                      : plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float)
+                                        : 0;
   void* ws = nullptr;
+  unsigned* counters = nullptr;
   if (a_sz + b_sz + p_sz > 0) {
-    const int rc = get_scratch(sc, a_sz + b_sz + p_sz, &ws);
+    const int rc = get_scratch(sc, a_sz + b_sz + p_sz, &ws, plan.fused ? &counters : nullptr);
     if (rc != HCG_OK) return rc;
   }
   const uint16_t* a_use = static_cast<const uint16_t*>(A);
@@ -3078,12 +3122,14 @@ int run_tiled(const Scratch& sc, int dtype, const void* A, int64_t lda, const vo
     f.splits = (K + f.kchunk - 1) / f.kchunk;
     f.ws = reinterpret_cast<float*>(static_cast<char*>(ws) + a_sz + b_sz);
     f.ws_vec = N % 4 == 0;  // 16-byte partial rows (the workspace base is 256-byte aligned)
+    f.counters = counters;
+    f.ws_bytes = (int)p_sz;
   }
   const int rc = k_tail ? (dtype == HCG_F16 ? launch_dma<HCG_F16, false, true>(f, plan.shape, stream)
                                           : launch_dma<HCG_BF16, false, true>(f, plan.shape, stream))
                         : (dtype == HCG_F16 ? launch_dma<HCG_F16, false>(f, plan.shape, stream)
                                             : launch_dma<HCG_BF16, false>(f, plan.shape, stream));
-  if (rc != HCG_OK || f.splits == 1) return rc;
+  if (rc != HCG_OK || f.splits == 1 || f.counters != nullptr) return rc;
   return launch_reduce(f.ws, C, ldc, M, N, M, f.splits, aligned16(C) && ldc % 4 == 0, stream);
 }
 
