@@ -2478,9 +2478,13 @@ constexpr TileShape kTileShapes[] = {
     {64, 64, 2, 64, true, 1.26f, 0.183f, 0.261f},
     {64, 128, 1, 64, true, 1.89f, 0.263f, 0.366f},
     {128, 256, 1, 64, true, 4.32f, 0.484f, 0.828f},
+    // Transposed operands only (gemm_dma_kernel's four waves are ahead on
+    // row-major ones: 4096^3 bf16 98.5 us against 103.4).
+    {256, 256, 1, 32, true, 8.04f, 0.460f, 0.70f},
 };
 constexpr int kNumTileShapes = sizeof(kTileShapes) / sizeof(kTileShapes[0]);
 constexpr int kNarrowShape = 4;
+constexpr int kTransShape = 8;
 constexpr double kLaunchUs = 2.0;
 
 // Picks the tile shape and K split with the least modelled time.
@@ -2549,10 +2553,12 @@ double plan_cost(const TileShape& t, int splits, bool fused, int num_cus, int M,
   return us;
 }
 
-// wide: operands that need gemm_dma_kernel's WIDE form (no wg8 shape has
-// one).  fuse: the caller's scratch has arrival counters.
+// kWide: operands that need gemm_dma_kernel's WIDE form (no wg8 shape has
+// one); kTrans: a transposed operand (only wg8 shapes read it).  fuse: the
+// caller's scratch has arrival counters.
+enum Operands { kRowMajor, kWide, kTrans };
 TilePlan plan_tiles(int num_cus, int M, int N, int K, int force_shape, bool allow_split, double* cost_out = nullptr,
-                    size_t room = kMaxSplitWorkspace, bool wide = false, bool fuse = true) {
+                    size_t room = kMaxSplitWorkspace, Operands ops = kRowMajor, bool fuse = true) {
   TilePlan best{force_shape >= 0 ? force_shape : 0, 1, false};
   double best_cost = -1;
   const int forced_splits =
@@ -2562,7 +2568,7 @@ TilePlan plan_tiles(int num_cus, int M, int N, int K, int force_shape, bool allo
   for (int i = 0; i < kNumTileShapes; ++i) {
     const TileShape& t = kTileShapes[i];
     if (force_shape >= 0 ? i != force_shape : i == kNarrowShape && N > 64) continue;
-    if (wide && force_shape < 0 && t.wg8) continue;
+    if (force_shape < 0 && (ops == kWide ? t.wg8 : ops == kTrans ? !t.wg8 : i == kTransShape)) continue;
     if (plan_tile_count(t, M, N) * 64 > 0x7fffffff) continue;
     for (int c = 0; c < (forced_splits > 0 ? 1 : (int)(sizeof(kSplitCandidates) / sizeof(int))); ++c) {
       const int splits = forced_splits > 0 ? forced_splits : kSplitCandidates[c];
@@ -2581,8 +2587,30 @@ TilePlan plan_tiles(int num_cus, int M, int N, int K, int force_shape, bool allo
   return best;
 }
 
-template <int DT, bool KT>
-int launch_wg8(const FastArgs& f, int shape, hipStream_t stream) {
+// AKC, BKC: the operand is K-contiguous (A as bound, B transposed).
+template <int DT, bool AKC, bool BKC, bool KT>
+int launch_wg8(const hcg::wg8::Args& a, int shape, hipStream_t stream) {
+  using namespace hcg::wg8;
+  const dim3 grid((unsigned)(a.tiles_m * a.tiles_n * a.splits));
+  const dim3 block(kThreads);
+  HCG_STAMP_ARGS(Args, a)
+  switch (shape) {
+    case 3: gemm_wg8_kernel<DT, 128, 128, 2, 2, 64, 4, AKC, BKC, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
+    case 5: gemm_wg8_kernel<DT, 64, 64, 2, 2, 64, 4, AKC, BKC, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
+    case 6: gemm_wg8_kernel<DT, 64, 128, 2, 2, 64, 4, AKC, BKC, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
+    case 7: gemm_wg8_kernel<DT, 128, 256, 2, 4, 64, 3, AKC, BKC, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
+    case kTransShape:
+      if constexpr (!(AKC && !BKC)) {
+        gemm_wg8_kernel<DT, 256, 256, 2, 4, 32, 4, AKC, BKC, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a));
+        break;
+      }
+    default: return set_error(HCG_EINVAL, "internal: shape %d", shape);
+  }
+  HCG_HIP_CHECK(hipGetLastError());
+  return HCG_OK;
+}
+
+hcg::wg8::Args wg8_args(const FastArgs& f) {
   hcg::wg8::Args a{};
   a.A = f.A;
   a.B = f.B;
@@ -2604,24 +2632,13 @@ int launch_wg8(const FastArgs& f, int shape, hipStream_t stream) {
   a.ws_vec = f.ws_vec;
   a.counters = f.counters;
   a.ws_bytes = f.ws_bytes;
-  const dim3 grid((unsigned)(a.tiles_m * a.tiles_n * a.splits));
-  const dim3 block(hcg::wg8::kThreads);
-  HCG_STAMP_ARGS(hcg::wg8::Args, a)
-  using namespace hcg::wg8;
-  switch (shape) {
-    case 3: gemm_wg8_kernel<DT, 128, 128, 2, 2, 64, 4, true, false, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
-    case 5: gemm_wg8_kernel<DT, 64, 64, 2, 2, 64, 4, true, false, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
-    case 6: gemm_wg8_kernel<DT, 64, 128, 2, 2, 64, 4, true, false, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
-    default: gemm_wg8_kernel<DT, 128, 256, 2, 4, 64, 3, true, false, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
-  }
-  HCG_HIP_CHECK(hipGetLastError());
-  return HCG_OK;
+  return a;
 }
 
 template <int DT, bool WIDE, bool KT = false>
 int launch_dma(const FastArgs& a, int shape, hipStream_t stream) {
   if constexpr (!WIDE) {
-    if (kTileShapes[shape].wg8) return launch_wg8<DT, KT>(a, shape, stream);
+    if (kTileShapes[shape].wg8) return launch_wg8<DT, true, false, KT>(wg8_args(a), shape, stream);
   }
   const dim3 grid((unsigned)(a.tiles_m * a.tiles_n * (a.splits > 1 ? a.splits : 1)));
   const dim3 block(kTiledThreads);
@@ -3039,7 +3056,7 @@ int run_tiled(const Scratch& sc, int dtype, const void* A, int64_t lda, const vo
                     (int64_t)kDmaK * ldb * 2 < kLimit && tiles <= 0x7fffffff;
   if (force_generic || (!fits && !wide)) return run_generic(dtype, A, lda, B, ldb, C, ldc, M, N, K, stream);
   if (wide) {
-    const TilePlan plan = plan_tiles(st->num_cus, M, N, K, force_shape, false, nullptr, 0, true);
+    const TilePlan plan = plan_tiles(st->num_cus, M, N, K, force_shape, false, nullptr, 0, kWide);
     const TileShape& ts = kTileShapes[plan.shape];
     FastArgs f{};
     f.A = static_cast<const uint16_t*>(A);
@@ -3064,7 +3081,7 @@ int run_tiled(const Scratch& sc, int dtype, const void* A, int64_t lda, const vo
   const size_t b_sz = b_ok ? 0 : round_up((size_t)K * ldb_p * 2, 256);
   // Explicit tile shapes run without a K split; "auto" and "tiled" may split.
   const TilePlan plan = plan_tiles(st->num_cus, M, N, K, force_shape, force_shape < 0, nullptr,
-                                   sc.room(a_sz + b_sz), false, sc.fixed == nullptr);
+                                   sc.room(a_sz + b_sz), kRowMajor, sc.fixed == nullptr);
   const TileShape& ts = kTileShapes[plan.shape];
   if ((int64_t)((M + ts.tm - 1) / ts.tm) * ((N + ts.tn - 1) / ts.tn) * plan.splits > 0x7fffffff)
     return run_generic(dtype, A, lda, B, ldb, C, ldc, M, N, K, stream);
@@ -3131,6 +3148,75 @@ int run_tiled(const Scratch& sc, int dtype, const void* A, int64_t lda, const vo
                                             : launch_dma<HCG_BF16, false>(f, plan.shape, stream));
   if (rc != HCG_OK || f.splits == 1 || f.counters != nullptr) return rc;
   return launch_reduce(f.ws, C, ldc, M, N, M, f.splits, aligned16(C) && ldc % 4 == 0, stream);
+}
+
+// The tiled kernel on a transposed operand, read where it lies: A stored as
+// K x M (a_t) or B stored as N x K (b_t), not both.  HCG_EDECLINED, with
+// nothing launched, for what only the row-major kernels take: few rows or
+// columns (streaming kernels), operands whose last 16-byte piece cannot be
+// read safely, offsets past 2^31.
+int run_trans(const Scratch& sc, int dtype, bool a_t, const void* A, int64_t lda, bool b_t, const void* B,
+              int64_t ldb, float* C, int64_t ldc, int64_t M, int64_t N, int64_t K) {
+  const int64_t kLimit = (int64_t)1 << 31;
+  const auto extent = [](int64_t rows, int64_t cols, int64_t ld) {
+    return ((int64_t)round_up(rows, 256) * ld + (int64_t)round_up(cols, 256) + 8) * 2;
+  };
+  // Stored rows and columns.
+  const int64_t ar = a_t ? K : M, ac = a_t ? M : K, br = b_t ? N : K, bc = b_t ? K : N;
+  if (a_t == b_t || M <= 64 || N <= 64 || lda >= kLimit || ldb >= kLimit || extent(ar, ac, lda) >= kLimit ||
+      extent(br, bc, ldb) >= kLimit)
+    return HCG_EDECLINED;
+  const bool k8 = K % 8 == 0;
+  const auto readable = [&](const void* p, int64_t rows, int64_t cols, int64_t ld, bool k_contig) {
+    return (aligned16(p) && ld % 8 == 0 && (k8 || !k_contig)) ||
+           (aligned2(p) && chunk_tail_readable(p, rows, cols, ld));
+  };
+  if (!readable(A, ar, ac, lda, !a_t) || !readable(B, br, bc, ldb, b_t)) return HCG_EDECLINED;
+  const TilePlan plan = plan_tiles(sc.st->num_cus, (int)M, (int)N, (int)K, -1, true, nullptr, sc.room(0), kTrans);
+  const TileShape& ts = kTileShapes[plan.shape];
+  hcg::wg8::Args a{};
+  a.A = static_cast<const uint16_t*>(A);
+  a.B = static_cast<const uint16_t*>(B);
+  a.C = C;
+  a.lda = (int)lda;
+  a.ldb = (int)ldb;
+  a.ldc = ldc;
+  a.M = (int)M;
+  a.N = (int)N;
+  a.K = (int)K;
+  a.tiles_m = (int)((M + ts.tm - 1) / ts.tm);
+  a.tiles_n = (int)((N + ts.tn - 1) / ts.tn);
+  if ((int64_t)a.tiles_m * a.tiles_n * plan.splits > 0x7fffffff) return HCG_EDECLINED;
+  // Extents end with the chunk that holds the last element.
+  a.a_bytes = (int)(((ar - 1) * lda + (int64_t)round_up(ac, 8)) * 2);
+  a.b_bytes = (int)(((br - 1) * ldb + (int64_t)round_up(bc, 8)) * 2);
+  a.c_vec = aligned16(C) && ldc % 4 == 0;
+  a.splits = 1;
+  if (plan.splits > 1) {
+    const int nk = (int)((K + ts.ks - 1) / ts.ks);
+    a.kchunk = (nk + plan.splits - 1) / plan.splits * ts.ks;
+    a.splits = (int)((K + a.kchunk - 1) / a.kchunk);
+    const size_t bytes = plan.fused ? fused_bytes(ts, plan.splits, (int)M, (int)N)
+                                    : (size_t)plan.splits * M * N * sizeof(float);
+    void* ws = nullptr;
+    const int rc = get_scratch(sc, bytes, &ws, plan.fused ? &a.counters : nullptr);
+    if (rc != HCG_OK) return rc;
+    a.ws = static_cast<float*>(ws);
+    a.ws_vec = N % 4 == 0;
+    if (a.counters) a.ws_bytes = (int)bytes;
+  }
+  int rc;
+  if (a_t)
+    rc = dtype == HCG_F16 ? launch_wg8<HCG_F16, false, false, false>(a, plan.shape, sc.stream)
+                          : launch_wg8<HCG_BF16, false, false, false>(a, plan.shape, sc.stream);
+  else if (k8)
+    rc = dtype == HCG_F16 ? launch_wg8<HCG_F16, true, true, false>(a, plan.shape, sc.stream)
+                          : launch_wg8<HCG_BF16, true, true, false>(a, plan.shape, sc.stream);
+  else
+    rc = dtype == HCG_F16 ? launch_wg8<HCG_F16, true, true, true>(a, plan.shape, sc.stream)
+                          : launch_wg8<HCG_BF16, true, true, true>(a, plan.shape, sc.stream);
+  if (rc != HCG_OK || a.splits == 1 || a.counters) return rc;
+  return launch_reduce(a.ws, C, ldc, (int)M, (int)N, (int)M, a.splits, a.c_vec, sc.stream);
 }
 
 // Remainder peeling (HCG_ALGO_AUTO only).  A few rows or columns past a
@@ -3322,6 +3408,31 @@ int hcg_gemm_algo(int algo, int dtype, const void* A, int64_t lda, const void* B
 int hcg_gemm_noalloc(int dtype, const void* A, int64_t lda, const void* B, int64_t ldb, float* C,
                      int64_t ldc, int64_t M, int64_t N, int64_t K, void* stream) {
   return gemm_impl(HCG_ALGO_AUTO, dtype, A, lda, B, ldb, C, ldc, M, N, K, stream, true);
+}
+
+int hcg_gemm_trans(int dtype, int a_trans, const void* A, int64_t lda, int b_trans, const void* B, int64_t ldb,
+                   float* C, int64_t ldc, int64_t M, int64_t N, int64_t K, void* stream) {
+  if (dtype != HCG_F16 && dtype != HCG_BF16)
+    return set_error(HCG_EINVAL, "dtype must be HCG_F16 (0) or HCG_BF16 (1), got %d", dtype);
+  const int64_t kMaxExtent = (int64_t)1 << 30;
+  if (M < 0 || N < 0 || K < 0 || M > kMaxExtent || N > kMaxExtent || K > kMaxExtent)
+    return set_error(HCG_EINVAL, "extent outside 0 .. 2^30: M=%lld N=%lld K=%lld", (long long)M, (long long)N,
+                     (long long)K);
+  t_last_error.clear();
+  if (M == 0 || N == 0) return HCG_OK;
+  if (K == 0) return HCG_EDECLINED;
+  if (A == nullptr || B == nullptr || C == nullptr) return set_error(HCG_EINVAL, "A, B or C is NULL");
+  if (lda < (a_trans ? M : K)) return set_error(HCG_EINVAL, "lda (%lld) below A's stored columns", (long long)lda);
+  if (ldb < (b_trans ? K : N)) return set_error(HCG_EINVAL, "ldb (%lld) below B's stored columns", (long long)ldb);
+  if (ldc < N) return set_error(HCG_EINVAL, "ldc (%lld) < N (%lld)", (long long)ldc, (long long)N);
+  DeviceState* st = nullptr;
+  const int rc = current_device_state(&st);
+  if (rc != HCG_OK) return rc;
+  Scratch sc;
+  sc.st = st;
+  sc.stream = static_cast<hipStream_t>(stream);
+  std::lock_guard<std::mutex> lock(st->ws_mutex);  // (see gemm_impl)
+  return run_trans(sc, dtype, a_trans != 0, A, lda, b_trans != 0, B, ldb, C, ldc, M, N, K);
 }
 
 const char* hcg_last_error(void) { return t_last_error.c_str(); }

@@ -27,6 +27,7 @@ kernel's name plays no part.
 
 from __future__ import annotations
 
+import contextlib
 import functools
 import os
 from collections.abc import Callable
@@ -334,6 +335,22 @@ def _gemm_torch(torch: Any, a: Any, b: Any, out: Any | None, algo: int) -> Any:
     if m == 0 or n == 0:
         return out
     sa, sb, so = a.stride(), b.stride(), out.stride()
+    if (algo == _native.HCG_ALGO_AUTO or algo == _native.HCG_ALGO_TILED) and m > 64 and n > 64 and k > 1:
+        # One operand a transposed view (x @ w.t(), x.t() @ dy): the tiled
+        # kernel reads it where it lies.
+        at = sa[0] == 1 and sa[1] >= m
+        bt = sb[0] == 1 and sb[1] >= k
+        if at != bt and (at or (sa[1] == 1 and sa[0] >= k)) and (bt or (sb[1] == 1 and sb[0] >= n)) \
+                and so[1] == 1 and so[0] >= n:
+            lib = _native.lib()
+            guard = contextlib.nullcontext() if _current_device(torch) == index else torch.cuda.device(index)
+            with guard:
+                rc = lib.hcg_gemm_trans(dtype, at, a.data_ptr(), sa[1] if at else sa[0], bt, b.data_ptr(),
+                                        sb[1] if bt else sb[0], out.data_ptr(), so[0], m, n, k,
+                                        _current_stream(torch, index) or None)
+            if rc != _native.HCG_EDECLINED:
+                _native.check(lib, rc, "hcg_gemm_trans")
+                return out
     if k > 0 and (sa[1] != 1 or (m > 1 and sa[0] < k)):
         a = a.contiguous()
         sa = a.stride()

@@ -23,6 +23,7 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
 HCG_OK = 0
 HCG_EINVAL = 1
 HCG_EHIP = 2
+HCG_EDECLINED = 3
 
 HCG_F16 = 0
 HCG_BF16 = 1
@@ -52,7 +53,7 @@ ALGOS = {
 }
 
 # Every symbol include/hcg_gemm.h, include/hcg_tile_ops.h and include/hcg_mfma.h declare.
-EXPORTS = ("hcg_init", "hcg_gemm", "hcg_gemm_algo", "hcg_gemm_noalloc", "hcg_last_error", "hcg_version",
+EXPORTS = ("hcg_init", "hcg_gemm", "hcg_gemm_algo", "hcg_gemm_noalloc", "hcg_gemm_trans", "hcg_last_error", "hcg_version",
            "hcg_operand_in_place", "hcg_tile_load", "hcg_tile_store", "hcg_mfma_step")
 
 NOALLOC_SCRATCH_BYTES = 32 << 20  # HCG_NOALLOC_SCRATCH_BYTES
@@ -73,6 +74,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.hcg_gemm_algo.restype = c_int
     lib.hcg_gemm_noalloc.argtypes = [c_int, vp, i64, vp, i64, vp, i64, i64, i64, i64, vp]
     lib.hcg_gemm_noalloc.restype = c_int
+    lib.hcg_gemm_trans.argtypes = [c_int, c_int, vp, i64, c_int, vp, i64, vp, i64, i64, i64, i64, vp]
+    lib.hcg_gemm_trans.restype = c_int
     lib.hcg_last_error.argtypes = []
     lib.hcg_last_error.restype = ctypes.c_char_p
     lib.hcg_version.argtypes = []

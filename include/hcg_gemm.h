@@ -40,6 +40,7 @@ extern "C" {
 #define HCG_OK 0
 #define HCG_EINVAL 1
 #define HCG_EHIP 2
+#define HCG_EDECLINED 3 /* hcg_gemm_trans only: nothing launched, use a row-major copy */
 
 /* Operand element types. */
 #define HCG_F16 0
@@ -101,6 +102,18 @@ int hcg_gemm_algo(int algo, int dtype, const void* A, int64_t lda, const void* B
  * every byte a call reads was written earlier in the same call. */
 int hcg_gemm_noalloc(int dtype, const void* A, int64_t lda, const void* B, int64_t ldb, float* C,
                      int64_t ldc, int64_t M, int64_t N, int64_t K, void* stream);
+
+/* C = A @ B with one operand stored transposed and read where it lies: with
+ * a_trans element (i,k) of A is A[k*lda + i] (A stored K x M), with b_trans
+ * element (k,j) of B is B[j*ldb + k] (B stored N x K).  The two products of a
+ * linear layer's backward, dX = dY @ W^T and dW = X^T @ dY, run without a
+ * transposing copy.  HCG_EDECLINED, with nothing launched and no error text,
+ * when the call needs a row-major copy instead: both or neither operand
+ * transposed, M <= 64 or N <= 64 (the streaming kernels'), K == 0, an operand
+ * whose last 16-byte piece cannot be read safely, or offsets past 2^31.  No
+ * counterpart in the reference, whose buffers are row-major. */
+int hcg_gemm_trans(int dtype, int a_trans, const void* A, int64_t lda, int b_trans, const void* B, int64_t ldb,
+                   float* C, int64_t ldc, int64_t M, int64_t N, int64_t K, void* stream);
 
 /* Text of the calling thread's last error ("" if none). */
 const char* hcg_last_error(void);

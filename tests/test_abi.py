@@ -222,3 +222,23 @@ def test_stamps_buffer_splits_into_two_consecutive_launches():
     (prev, prev_wg), (last, last_wg) = stamps.split_launches(buf)
     assert list(prev_wg) == [0, 1, 2] and list(last_wg) == [0, 2]
     assert int(prev[:, 3].max()) == 1900 and int(last[:, 0].min()) == 2000
+
+
+@pytest.mark.parametrize("args,match", [
+    ((2, 0, 1, 8, 1, 1, 8, 1, 8, 8, 8, 8, None), "dtype"),
+    ((0, 0, 1, 8, 1, 1, 8, 1, 8, -1, 8, 8, None), "extent"),
+    ((0, 0, None, 128, 1, 1, 128, 1, 128, 128, 128, 128, None), "NULL"),
+    ((0, 1, 1, 127, 0, 1, 128, 1, 128, 128, 128, 64, None), "lda"),
+    ((0, 0, 1, 64, 1, 1, 63, 1, 128, 128, 128, 64, None), "ldb"),
+    ((0, 0, 1, 64, 1, 1, 64, 1, 127, 128, 128, 64, None), "ldc"),
+])
+def test_trans_rejects_bad_arguments_on_the_host(args, match):
+    lib = _native.load()
+    assert lib.hcg_gemm_trans(*args) == _native.HCG_EINVAL
+    assert match in _native.last_error(lib)
+
+
+def test_trans_with_nothing_to_do_launches_nothing():
+    lib = _native.load()
+    assert lib.hcg_gemm_trans(0, 1, None, 0, 0, None, 0, None, 0, 0, 8, 8, None) == _native.HCG_OK
+    assert lib.hcg_gemm_trans(0, 1, 1, 128, 0, 1, 128, 1, 128, 128, 128, 0, None) == _native.HCG_EDECLINED

@@ -76,3 +76,68 @@ def test_wg8_split_k(m, n, k):
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (128, 128, 31), (129, 257, 96), (640, 384, 1000)])
 def test_forced_128x128(m, n, k):
     _check(m, n, k, "float16", 4, "tiled_128x128")
+
+
+# A transposed operand is read where it lies; the padding of its stored rows
+# (past M for A stored K x M, past K for B stored N x K) holds NaN.
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("which", ["a", "b"])
+@pytest.mark.parametrize("m,n,k", [(65, 65, 2), (130, 100, 63), (127, 129, 64), (129, 190, 257), (200, 8192, 1000),
+                                   (1601, 2041, 264), (2500, 2500, 1001), (4095, 3001, 100), (4096, 4096, 72),
+                                   (512, 512, 4104), (333, 444, 4999)])
+@pytest.mark.parametrize("pad", [0, 3, 8])
+def test_transposed_operand_in_place(m, n, k, which, dtype, pad):
+    import hc.gfx950 as g
+
+    print(f"case transposed {which} {dtype} m={m} n={n} k={k} pad={pad}", flush=True)
+    rng = np.random.default_rng(m + 3 * n + 7 * k)
+    ai, bi = rng.integers(-4, 5, size=(m, k)), rng.integers(-4, 5, size=(k, n))
+    a = _padded(ai.T, DTYPES[dtype], pad).t() if which == "a" else _padded(ai, DTYPES[dtype], pad)
+    b = _padded(bi.T, DTYPES[dtype], pad).t() if which == "b" else _padded(bi, DTYPES[dtype], pad)
+    guard = torch.full((m + 2, n + 5), float("nan"), dtype=torch.float32, device=DEV)
+    g.gemm(a, b, out=guard[:m, :n])
+    torch.cuda.synchronize()
+    got = guard.cpu().numpy()
+    want = (ai.astype(np.float64) @ bi.astype(np.float64)).astype(np.float32)
+    assert np.array_equal(got[:m, :n], want)
+    assert np.all(np.isnan(got[m:])) and np.all(np.isnan(got[:, n:]))
+    assert torch.equal(g.gemm(a, b), torch.from_numpy(want).to(DEV))  # without out=
+
+
+@pytest.mark.parametrize("m,n,k", [(64, 200, 96), (200, 64, 96), (3, 70, 8), (70, 70, 1), (100, 100, 40)])
+def test_transposed_operands_the_kernel_declines_are_copied(m, n, k):
+    """Few rows or columns, K = 1, and both operands transposed take the
+    row-major path on copies."""
+    import hc.gfx950 as g
+
+    rng = np.random.default_rng(m + n + k)
+    ai, bi = rng.integers(-4, 5, size=(m, k)), rng.integers(-4, 5, size=(k, n))
+    a, b = _padded(ai, torch.float16, 1), _padded(bi, torch.float16, 1)
+    at, bt = _padded(ai.T, torch.float16, 1).t(), _padded(bi.T, torch.float16, 1).t()
+    want = torch.from_numpy((ai.astype(np.float64) @ bi.astype(np.float64)).astype(np.float32)).to(DEV)
+    for x, y in ((at, bt), (at, b), (a, bt)):
+        assert torch.equal(g.gemm(x, y), want)
+
+
+def test_transposed_operand_under_capture():
+    """A split-K call on a transposed operand replays from a graph, with eager
+    calls between the replays, and repeats bit for bit."""
+    import hc.gfx950 as g
+
+    x = torch.randn(8192, 300, device=DEV).half()
+    dy = torch.randn(8192, 200, device=DEV).half()
+    out = torch.empty(300, 200, device=DEV)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        g.gemm(x.t(), dy, out=out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        g.gemm(x.t(), dy, out=out)
+    for _ in range(4):
+        x.copy_(torch.randn_like(x))
+        eager = g.gemm(x.t(), dy)
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
