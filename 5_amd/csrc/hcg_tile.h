@@ -12,10 +12,10 @@
 // On gfx950 these become bounds-predicated vector accesses: an element
 // outside the extent is never read (its payload is the fill value) and
 // never written.  Two forms are provided:
-//   * row-chunk loads/stores through plain pointers (up to 8 consecutive
-//     elements of one row, one 16-byte access when the chunk is whole and
-//     aligned, element accesses at the edges), used by register-staged
-//     kernels and the tile gather/scatter entry points;
+//   * row-chunk loads through plain pointers (up to 8 consecutive elements
+//     of one row, one 16-byte access when the chunk is whole and aligned,
+//     element accesses at the edges), used by register-staged kernels, and a
+//     chunk's activity bits, used by the tile gather/scatter entry points;
 //   * buffer-resource DMA into LDS (buffer_load ... lds), where the
 //     hardware range check returns zeros for offsets at or beyond the
 //     extent and a per-lane redirect (dma_offset) sends chunks that are out
@@ -67,43 +67,6 @@ __device__ __forceinline__ uint32_t chunk_active_bits(int64_t row, int64_t nrows
     if (c >= 0 && c < ncols) bits |= 1u << e;
   }
   return bits;
-}
-
-// Loads the n (<= 8) elements of T at rowp[col0 + e] whose bit is set in
-// `active` (one vector access when all n are active and the chunk is
-// 16-byte aligned); others get `fill`.
-template <typename T>
-__device__ __forceinline__ void load_chunk(const T* rowp, int64_t col0, int n, uint32_t active, T fill,
-                                           T (&out)[8]) {
-  const T* p = rowp + col0;
-  const bool whole = n * sizeof(T) == 16 && active == (1u << n) - 1u &&
-                     (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
-  if (whole) {
-    const u32x4 v = *reinterpret_cast<const u32x4*>(p);
-    __builtin_memcpy(out, &v, 16);
-    return;
-  }
-#pragma unroll
-  for (int e = 0; e < 8; ++e) out[e] = (e < n && ((active >> e) & 1u)) ? p[e] : fill;
-}
-
-// Stores the elements of `v` whose bit is set in `write` to rowp[col0 + e]
-// (one vector access when all n are written and the chunk is 16-byte
-// aligned); nothing else is touched.
-template <typename T>
-__device__ __forceinline__ void store_chunk(T* rowp, int64_t col0, int n, uint32_t write, const T (&v)[8]) {
-  T* p = rowp + col0;
-  const bool whole = n * sizeof(T) == 16 && write == (1u << n) - 1u &&
-                     (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
-  if (whole) {
-    u32x4 w;
-    __builtin_memcpy(&w, v, 16);
-    *reinterpret_cast<u32x4*>(p) = w;
-    return;
-  }
-#pragma unroll
-  for (int e = 0; e < 8; ++e)
-    if (e < n && ((write >> e) & 1u)) p[e] = v[e];
 }
 
 // ---------------------------------------------------------------------------

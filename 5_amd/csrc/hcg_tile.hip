@@ -9,14 +9,24 @@
 // _store_from_value: only active elements inside the target view are
 // written), doc/langref.md:530-596 (masking, with_inactive, .mask).
 //
-// One thread handles one chunk of 16 bytes of one tile row (8, 4 or 2
-// elements); chunks wholly inside the source row and 16-byte aligned move
-// as one vector access, edge chunks element by element, and elements
-// outside the view are never read or written.
+// Bound: HBM (copies).  One thread moves one chunk of 16 bytes of one tile
+// row (8, 4 or 2 elements): a chunk wholly inside the view moves as one
+// vector access at the elements' own alignment (rows of a view need not be
+// 16-byte aligned, and gfx950 takes unaligned global accesses), its activity
+// as one word; edge chunks go element by element, and elements outside the
+// view are never read or written.  Per-element accesses for rows that are not
+// 16-byte aligned, byte stores of the activity and 64-bit divisions per chunk
+// made the form before this one instruction-bound: the 64x64 tiles of a tight
+// 4095 x 3001 f16 matrix (61 MB each way) gather in 21.0 -> 14.8 us and scatter
+// in 29.6 -> 16.4, and in 11.4 and 15.0 with each XCD on neighbouring tiles
+// (block_of).  Four chunks per thread, all loads first, did not help (16.0 and
+// 17.4 without the mapping): latency is covered by the waves in flight.
 
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "hcg_runtime.h"
 #include "hcg_tile.h"
@@ -40,69 +50,165 @@ struct TileJob {
   uint64_t fill_bits;      // load: with_inactive value, low sizeof(T) bytes
 };
 
-template <typename T>
-__device__ __forceinline__ void decompose(const TileJob& j, int64_t idx, int64_t& t, int64_t& r, int64_t& c0) {
-  const int64_t row_id = idx / j.chunks_per_row;  // t * th + r
-  c0 = (idx - row_id * j.chunks_per_row) * (16 / (int64_t)sizeof(T));
-  t = row_id / j.th;
-  r = row_id - t * j.th;
+// Chunk index -> tile, row and first column in the tile.  I: uint32_t when
+// every index fits (a 64-bit division costs about as much as the rest of a
+// chunk's work), else int64_t.
+template <typename T, typename I>
+__device__ __forceinline__ void decompose(const TileJob& j, I idx, int64_t& t, int64_t& r, int64_t& c0) {
+  const I per = (I)j.chunks_per_row, th = (I)j.th;
+  const I row_id = idx / per;  // t * th + r
+  const I tile = row_id / th;
+  c0 = (int64_t)(idx - row_id * per) * (16 / (int64_t)sizeof(T));
+  t = (int64_t)tile;
+  r = (int64_t)(row_id - tile * th);
 }
 
+// 16 bytes, and one byte per element of a chunk, at element alignment.
 template <typename T>
+struct Chunk {
+  static constexpr int kN = 16 / sizeof(T);
+  union {
+    hcg::u32x4 v;
+    T e[kN];
+  };
+  // Activity bytes of a chunk (kN of 8, 4 or 2 bytes).
+  typedef std::conditional_t<kN == 8, uint64_t, std::conditional_t<kN == 4, uint32_t, uint16_t>> Bytes;
+
+  __device__ __forceinline__ void load(const T* p) { __builtin_memcpy(&v, p, 16); }
+  __device__ __forceinline__ void store(T* p) const { __builtin_memcpy(p, &v, 16); }
+};
+
+// Bits of the elements whose activity byte is nonzero.
+template <typename T>
+__device__ __forceinline__ uint32_t mask_bits(const uint8_t* m, int n) {
+  constexpr int kN = Chunk<T>::kN;
+  uint32_t bits = 0;
+  if (n == kN) {
+    typename Chunk<T>::Bytes b;
+    __builtin_memcpy(&b, m, sizeof b);
+    const uint64_t w = b;
+#pragma unroll
+    for (int e = 0; e < kN; ++e) bits |= ((w >> (8 * e)) & 0xff) ? 1u << e : 0u;
+  } else {
+#pragma unroll
+    for (int e = 0; e < kN; ++e)
+      if (e < n && m[e]) bits |= 1u << e;
+  }
+  return bits;
+}
+
+// Workgroup -> block of 256 chunks: workgroups go round-robin over the 8 XCDs
+// (id % 8), so each XCD takes a contiguous run of blocks -- with rows that are
+// not line-aligned, neighbouring tiles share lines of the view, and one L2
+// then merges them.
+__device__ __forceinline__ int64_t block_of(unsigned wg, unsigned grid) {
+  const unsigned per = grid >> 3, rem = grid & 7, x = wg & 7, i = wg >> 3;
+  return x < rem ? (int64_t)x * (per + 1) + i : (int64_t)rem * (per + 1) + (int64_t)(x - rem) * per + i;
+}
+
+template <typename T, typename I>
 __global__ __launch_bounds__(256) void tile_load_kernel(TileJob j) {
-  constexpr int kN = 16 / sizeof(T);
+  constexpr int kN = Chunk<T>::kN;
+  constexpr uint32_t kAll = (1u << kN) - 1u;
   T fill;
   __builtin_memcpy(&fill, &j.fill_bits, sizeof(T));
-  for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < j.total_chunks;
-       idx += (int64_t)gridDim.x * 256) {
+  for (int64_t at = block_of(blockIdx.x, gridDim.x) * 256 + threadIdx.x; at < j.total_chunks;
+       at += (int64_t)gridDim.x * 256) {
     int64_t t, r, c0;
-    decompose<T>(j, idx, t, r, c0);
+    decompose<T, I>(j, (I)at, t, r, c0);
     const int n = (int)min((int64_t)kN, j.tw - c0);
     const int64_t row = j.origins[2 * t] + r;
     const int64_t col = j.origins[2 * t + 1] + c0;
     const int64_t out_off = (t * j.th + r) * j.tw + c0;
-    uint32_t active = hcg::chunk_active_bits(row, j.rows, col, j.cols, n);
-    if (j.mask_in) {
-#pragma unroll
-      for (int e = 0; e < kN; ++e)
-        if (e < n && j.mask_in[out_off + e] == 0) active &= ~(1u << e);
-    }
+    const bool whole = n == kN && row >= 0 && row < j.rows && col >= 0 && col + kN <= j.cols;
+    uint32_t active = whole ? kAll : hcg::chunk_active_bits(row, j.rows, col, j.cols, n);
+    if (j.mask_in) active &= mask_bits<T>(j.mask_in + out_off, n);
     // Rows outside the view are never addressed (active is 0 for them).
-    const T* rowp = static_cast<const T*>(j.src) + (active ? row * j.ld : 0);
-    T v[8];
-    hcg::load_chunk<T>(rowp, col, n, active, fill, v);
-    hcg::store_chunk<T>(static_cast<T*>(j.tiles_out) + (t * j.th + r) * j.tw, c0, n, (1u << n) - 1u, v);
-    if (j.mask_out) {
+    const T* p = static_cast<const T*>(j.src) + (active ? row * j.ld + col : 0);
+    Chunk<T> c;
+    if (whole && active) {
+      c.load(p);
+      if (active != kAll) {
+#pragma unroll
+        for (int e = 0; e < kN; ++e)
+          if (!((active >> e) & 1u)) c.e[e] = fill;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < kN; ++e) c.e[e] = ((active >> e) & 1u) ? p[e] : fill;
+    }
+    T* out = static_cast<T*>(j.tiles_out) + out_off;
+    uint8_t* om = j.mask_out ? j.mask_out + out_off : nullptr;
+    if (n == kN) {
+      c.store(out);
+      if (om) {
+        uint64_t w = 0;
+#pragma unroll
+        for (int e = 0; e < kN; ++e) w |= (uint64_t)((active >> e) & 1u) << (8 * e);
+        const typename Chunk<T>::Bytes b = (typename Chunk<T>::Bytes)w;
+        __builtin_memcpy(om, &b, sizeof b);
+      }
+    } else {
 #pragma unroll
       for (int e = 0; e < kN; ++e)
-        if (e < n) j.mask_out[out_off + e] = (active >> e) & 1u;
+        if (e < n) {
+          out[e] = c.e[e];
+          if (om) om[e] = (active >> e) & 1u;
+        }
+    }
+  }
+}
+
+template <typename T, typename I>
+__global__ __launch_bounds__(256) void tile_store_kernel(TileJob j) {
+  constexpr int kN = Chunk<T>::kN;
+  constexpr uint32_t kAll = (1u << kN) - 1u;
+  for (int64_t at = block_of(blockIdx.x, gridDim.x) * 256 + threadIdx.x; at < j.total_chunks;
+       at += (int64_t)gridDim.x * 256) {
+    int64_t t, r, c0;
+    decompose<T, I>(j, (I)at, t, r, c0);
+    const int n = (int)min((int64_t)kN, j.tw - c0);
+    const int64_t row = j.origins[2 * t] + r;
+    const int64_t col = j.origins[2 * t + 1] + c0;
+    const int64_t in_off = (t * j.th + r) * j.tw + c0;
+    const bool whole = n == kN && row >= 0 && row < j.rows && col >= 0 && col + kN <= j.cols;
+    uint32_t write = whole ? kAll : hcg::chunk_active_bits(row, j.rows, col, j.cols, n);
+    if (write == 0) continue;
+    const T* in = static_cast<const T*>(j.tiles_in) + in_off;
+    Chunk<T> c;
+    if (n == kN) {
+      c.load(in);  // beside the mask's load: a tile's chunk is always readable
+    } else {
+#pragma unroll
+      for (int e = 0; e < kN; ++e)
+        if (e < n) c.e[e] = in[e];
+    }
+    if (j.mask_in) write &= mask_bits<T>(j.mask_in + in_off, n);
+    if (write == 0) continue;
+    T* p = static_cast<T*>(j.dst) + row * j.ld + col;
+    if (write == kAll) {
+      c.store(p);
+    } else {
+#pragma unroll
+      for (int e = 0; e < kN; ++e)
+        if ((write >> e) & 1u) p[e] = c.e[e];
     }
   }
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void tile_store_kernel(TileJob j) {
-  constexpr int kN = 16 / sizeof(T);
-  for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < j.total_chunks;
-       idx += (int64_t)gridDim.x * 256) {
-    int64_t t, r, c0;
-    decompose<T>(j, idx, t, r, c0);
-    const int n = (int)min((int64_t)kN, j.tw - c0);
-    const int64_t row = j.origins[2 * t] + r;
-    const int64_t col = j.origins[2 * t + 1] + c0;
-    const int64_t in_off = (t * j.th + r) * j.tw + c0;
-    uint32_t write = hcg::chunk_active_bits(row, j.rows, col, j.cols, n);
-    if (j.mask_in) {
-#pragma unroll
-      for (int e = 0; e < kN; ++e)
-        if (e < n && j.mask_in[in_off + e] == 0) write &= ~(1u << e);
-    }
-    if (write == 0) continue;
-    T v[8];
-    hcg::load_chunk<T>(static_cast<const T*>(j.tiles_in) + (t * j.th + r) * j.tw, c0, n, (1u << n) - 1u, T{},
-                       v);
-    hcg::store_chunk<T>(static_cast<T*>(j.dst) + row * j.ld, col, n, write, v);
-  }
+void run_load(const TileJob& j, unsigned grid, hipStream_t s) {
+  if (j.total_chunks <= 0x7fffffff)
+    tile_load_kernel<T, uint32_t><<<grid, 256, 0, s>>>(j);
+  else
+    tile_load_kernel<T, int64_t><<<grid, 256, 0, s>>>(j);
+}
+template <typename T>
+void run_store(const TileJob& j, unsigned grid, hipStream_t s) {
+  if (j.total_chunks <= 0x7fffffff)
+    tile_store_kernel<T, uint32_t><<<grid, 256, 0, s>>>(j);
+  else
+    tile_store_kernel<T, int64_t><<<grid, 256, 0, s>>>(j);
 }
 
 // Argument checks shared by both entry points; fills the geometry of j.
@@ -161,11 +267,11 @@ int hcg_tile_load(int elem_bytes, const void* src, int64_t ld, int64_t rows, int
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const unsigned grid = grid_for(j.total_chunks);
   if (elem_bytes == 2)
-    tile_load_kernel<uint16_t><<<grid, 256, 0, s>>>(j);
+    run_load<uint16_t>(j, grid, s);
   else if (elem_bytes == 4)
-    tile_load_kernel<uint32_t><<<grid, 256, 0, s>>>(j);
+    run_load<uint32_t>(j, grid, s);
   else
-    tile_load_kernel<uint64_t><<<grid, 256, 0, s>>>(j);
+    run_load<uint64_t>(j, grid, s);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hcg::set_error(HCG_EHIP, "tile_load_kernel launch failed: %s", hipGetErrorString(e));
   hcg::t_last_error.clear();
@@ -189,11 +295,11 @@ int hcg_tile_store(int elem_bytes, void* dst, int64_t ld, int64_t rows, int64_t 
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const unsigned grid = grid_for(j.total_chunks);
   if (elem_bytes == 2)
-    tile_store_kernel<uint16_t><<<grid, 256, 0, s>>>(j);
+    run_store<uint16_t>(j, grid, s);
   else if (elem_bytes == 4)
-    tile_store_kernel<uint32_t><<<grid, 256, 0, s>>>(j);
+    run_store<uint32_t>(j, grid, s);
   else
-    tile_store_kernel<uint64_t><<<grid, 256, 0, s>>>(j);
+    run_store<uint64_t>(j, grid, s);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hcg::set_error(HCG_EHIP, "tile_store_kernel launch failed: %s", hipGetErrorString(e));
   hcg::t_last_error.clear();

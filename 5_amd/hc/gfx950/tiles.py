@@ -65,7 +65,7 @@ def _mask(torch: Any, mask: Any, shape: tuple[int, int, int], device: Any) -> An
         raise LaunchError(f"mask shape {tuple(m.shape)} does not match the tiles {shape}")
     if m.dtype != torch.bool and m.dtype != torch.uint8:
         raise LaunchError(f"mask= expects a bool tensor, got {m.dtype}")
-    return m.to(torch.uint8).contiguous()
+    return m.contiguous().view(torch.uint8)  # (a bool's byte is nonzero where true: no conversion pass)
 
 
 def _fill_bits(torch: Any, fill: Any, dtype: Any) -> int:

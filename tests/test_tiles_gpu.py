@@ -143,3 +143,25 @@ def test_tile_store_then_load_round_trip_bf16():
     a = act.cpu()
     assert torch.equal(back.cpu()[a], tiles.cpu()[a])
     assert a[0].all() and a[1].sum().item() == 17 * 7 and a[2].sum().item() == 17 * 7
+
+
+def test_more_chunks_than_one_pass_of_the_grid():
+    """Past 65536 workgroups of 256 chunks the grid strides: 290000 tiles of
+    16x16 float32 are 18.6 million chunks (297 MB of tiles)."""
+    import hc.gfx950 as g
+
+    rng = np.random.default_rng(5)
+    src = torch.arange(301 * 203, dtype=torch.float32, device=DEV).view(301, 203)
+    n = 290000
+    o = torch.from_numpy(np.stack([rng.integers(-8, 300, n), rng.integers(-8, 200, n)], axis=1)).to(DEV)
+    tiles, active = g.tile_load(src, o, (16, 16), fill=-1)
+    r = (o[:, 0:1] + torch.arange(16, device=DEV))[:, :, None].expand(n, 16, 16)
+    c = (o[:, 1:2] + torch.arange(16, device=DEV))[:, None, :].expand(n, 16, 16)
+    inside = (r >= 0) & (r < 301) & (c >= 0) & (c < 203)
+    assert torch.equal(active, inside)
+    assert torch.equal(tiles, torch.where(inside, (r * 203 + c).float(), torch.full_like(tiles, -1)))
+    dst = torch.zeros_like(src)
+    g.tile_store(dst, o, tiles, mask=active)
+    covered = torch.zeros_like(src, dtype=torch.bool)
+    covered[r[inside], c[inside]] = True
+    assert torch.equal(dst, torch.where(covered, src, torch.zeros_like(src)))
