@@ -13,9 +13,14 @@ Buffers may be ``numpy.ndarray`` (as in the reference) or ``torch.Tensor``
 
 from __future__ import annotations
 
+import functools
 import inspect
+import sys
 from dataclasses import dataclass
+from types import CodeType, FunctionType
 from typing import Any, get_args, get_origin
+
+import numpy as np
 
 from ._errors import LaunchError
 from .core import BufferSpec, KernelMetadata
@@ -38,22 +43,21 @@ class PreparedLaunch:
         return any(dim == 0 for dim in self.work_shape)
 
 
+_TORCH_DTYPE_NAMES: dict[Any, str] = {}  # torch dtype -> name (torch has a fixed set of them)
+
+
 def buffer_dtype_name(value: Any) -> str | None:
     """dtype name of a numpy array or torch tensor, else None."""
-    import numpy as np
-
     if isinstance(value, np.ndarray):
         return str(value.dtype.name)
-    torch = _torch_if_loaded()
+    torch = sys.modules.get("torch")
     if torch is not None and isinstance(value, torch.Tensor):
-        return str(value.dtype).replace("torch.", "")
+        dtype = value.dtype
+        name = _TORCH_DTYPE_NAMES.get(dtype)
+        if name is None:
+            name = _TORCH_DTYPE_NAMES[dtype] = str(dtype).replace("torch.", "")
+        return name
     return None
-
-
-def _torch_if_loaded() -> Any:
-    import sys
-
-    return sys.modules.get("torch")
 
 
 def is_buffer(value: Any) -> bool:
@@ -67,7 +71,32 @@ def kernel_metadata(fn: Any) -> KernelMetadata:
     return metadata
 
 
+class _PositionalBound(inspect.BoundArguments):
+    """Arguments bound by position; the signature is built when asked for."""
+
+    __slots__ = ("_fn",)
+
+    def __init__(self, fn: Any, arguments: dict[str, Any]) -> None:
+        self._fn = fn
+        self.arguments = arguments
+
+    @property
+    def _signature(self) -> inspect.Signature:
+        return inspect.Signature(list(inspect.signature(self._fn).parameters.values())[1:])
+
+
+_VARIADIC = inspect.CO_VARARGS | inspect.CO_VARKEYWORDS
+
+
 def _bind_arguments(fn: Any, args: tuple[Any, ...], kwargs: dict[str, Any]) -> inspect.BoundArguments:
+    # A plain function called with exactly its positional parameters (the
+    # usual launch) binds by name order, as inspect would: building a
+    # Signature takes longer than a small product.
+    if not kwargs and type(fn) is FunctionType and "__signature__" not in fn.__dict__ and "__wrapped__" not in fn.__dict__:
+        code = fn.__code__
+        count = code.co_argcount
+        if count == len(args) + 1 and not code.co_kwonlyargcount and not code.co_flags & _VARIADIC:
+            return _PositionalBound(fn, dict(zip(code.co_varnames[1:count], args)))
     params = list(inspect.signature(fn).parameters.values())
     if not params:
         raise LaunchError("kernel must accept a CurrentGroup parameter")
@@ -79,31 +108,46 @@ def _bind_arguments(fn: Any, args: tuple[Any, ...], kwargs: dict[str, Any]) -> i
 
 class _SymbolFallback(dict):
     """Evaluation namespace for string annotations: the kernel's closure
-    variables, then its globals, and any other capitalised name becomes the
-    symbol of that name (``Buffer["M", "K"]`` style annotations)."""
+    variables, then its globals (both as they are when a name is looked up),
+    and any other capitalised name becomes the symbol of that name
+    (``Buffer["M", "K"]`` style annotations)."""
 
     def __init__(self, fn: Any) -> None:
-        super().__init__(fn.__globals__)
-        self.update(inspect.getclosurevars(fn).nonlocals)
+        if type(fn) is FunctionType:
+            if fn.__closure__:
+                super().__init__(zip(fn.__code__.co_freevars, [cell.cell_contents for cell in fn.__closure__]))
+        else:
+            super().__init__(inspect.getclosurevars(fn).nonlocals)
+        self._globals = fn.__globals__
 
     def __missing__(self, name: str) -> Any:
+        try:
+            return self._globals[name]
+        except KeyError:
+            pass
         if not name[:1].isupper():
             raise KeyError(name)
         return getattr(sym, name)
 
 
+@functools.lru_cache(maxsize=512)
+def _annotation_code(text: str) -> CodeType:
+    """``text`` compiled; what its names mean is looked up at every evaluation."""
+    return compile(text.lstrip(" \t"), "<annotation>", "eval")
+
+
 def resolved_annotations(fn: Any) -> dict[str, Any]:
     """The kernel's parameter annotations with string annotations evaluated
     (hc/simulator.py:664-700 semantics)."""
-    raw = inspect.get_annotations(fn, eval_str=False)
-    pending = {name: text for name, text in raw.items() if isinstance(text, str)}
-    if not pending:
-        return dict(raw)
-    namespace = _SymbolFallback(fn)
-    out = dict(raw)
-    for name, text in pending.items():
+    out = dict(fn.__annotations__) if type(fn) is FunctionType else dict(inspect.get_annotations(fn, eval_str=False))
+    namespace = None
+    for name, text in out.items():
+        if not isinstance(text, str):
+            continue
+        if namespace is None:
+            namespace = _SymbolFallback(fn)
         try:
-            out[name] = eval(text, fn.__globals__, namespace)  # noqa: S307 - annotation text
+            out[name] = eval(_annotation_code(text), fn.__globals__, namespace)  # noqa: S307 - annotation text
         except (NameError, TypeError) as exc:
             raise LaunchError(f"failed to resolve annotations for {fn.__name__}") from exc
     return out
@@ -126,14 +170,19 @@ class _Binder:
             raise LaunchError(f"{where} expected {dim}, got {value}")
 
     def shape(self, dims: tuple[Any, ...], shape: tuple[int, ...], where: str) -> None:
+        bind = self.bindings.bind
         for index, (dim, value) in enumerate(zip(dims, shape)):
-            self.extent(dim, int(value), f"{where}.shape[{index}]")
+            source = f"{where}.shape[{index}]"
+            if type(dim) is Symbol:
+                bind(dim, int(value), source=source)
+            else:
+                self.extent(dim, int(value), source)
 
     def buffer(self, spec: BufferSpec, value: Any, where: str) -> None:
         dtype = buffer_dtype_name(value)
         if dtype is None:
             raise LaunchError(f"{where} must be a numpy.ndarray or torch.Tensor buffer")
-        shape = tuple(int(d) for d in value.shape)
+        shape = value.shape
         if len(shape) != len(spec.dimensions):
             raise LaunchError(f"{where} rank does not match its Buffer annotation")
         if spec.dtype is not None and dtype != spec.dtype:
@@ -150,8 +199,6 @@ class _Binder:
 
 
 def _resolve_dim(value: Any, env: Env, literal_names: frozenset[str], *, static: bool, name: str) -> int:
-    import numpy as np
-
     if isinstance(value, bool):
         raise LaunchError(f"{name} must be an integer")
     if isinstance(value, (int, np.integer)):

@@ -31,6 +31,8 @@ from collections.abc import Callable, Sequence
 from dataclasses import dataclass, field
 from typing import Any
 
+import numpy as np
+
 
 class _BFloat16:
     """Element-type marker for bfloat16 (no NumPy dtype exists for it)."""
@@ -47,21 +49,27 @@ bfloat16 = _BFloat16()
 def _dtype_name(value: Any) -> str:
     if value is bfloat16 or value == "bfloat16":
         return "bfloat16"
-    import numpy as np
-
     return str(np.dtype(value).name)
+
+
+# NumPy scalar type -> dtype name (asking np.dtype takes longer than the rest
+# of a Buffer annotation, which every launch evaluates).
+_SCALAR_NAMES = {t: str(np.dtype(t).name) for t in (np.float16, np.float32, np.float64, np.int8, np.int16, np.int32,
+                                                    np.int64, np.uint8, np.uint16, np.uint32, np.uint64, np.bool_)}
 
 
 def _buffer_dtype_name(value: Any) -> str | None:
     """Trailing Buffer[...] item -> dtype name, or None if it is a dimension."""
-    import numpy as np
-
     if value is bfloat16:
         return "bfloat16"
     if isinstance(value, np.dtype):
         return str(value.name)
-    if isinstance(value, type) and issubclass(value, np.generic):
-        return str(np.dtype(value).name)
+    if isinstance(value, type):
+        name = _SCALAR_NAMES.get(value)
+        if name is not None:
+            return name
+        if issubclass(value, np.generic):
+            return str(np.dtype(value).name)
     return None
 
 

@@ -159,7 +159,7 @@ def gemm(
 
 def tile_load(elem_bytes: int, src: int, ld: int, rows: int, cols: int, origins: int, ntiles: int, th: int,
               tw: int, in_mask: int, fill_bits: int, out: int, out_mask: int, stream: int) -> None:
-    lib = load()
+    lib = _lib if _lib is not None else load()
     rc = lib.hcg_tile_load(elem_bytes, src or None, ld, rows, cols, origins or None, ntiles, th, tw,
                            in_mask or None, fill_bits, out or None, out_mask or None, stream or None)
     check(lib, rc, "hcg_tile_load")
@@ -167,7 +167,7 @@ def tile_load(elem_bytes: int, src: int, ld: int, rows: int, cols: int, origins:
 
 def tile_store(elem_bytes: int, dst: int, ld: int, rows: int, cols: int, origins: int, ntiles: int, th: int,
                tw: int, tiles: int, tile_mask: int, stream: int) -> None:
-    lib = load()
+    lib = _lib if _lib is not None else load()
     rc = lib.hcg_tile_store(elem_bytes, dst or None, ld, rows, cols, origins or None, ntiles, th, tw,
                             tiles or None, tile_mask or None, stream or None)
     check(lib, rc, "hcg_tile_store")

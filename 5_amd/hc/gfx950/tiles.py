@@ -19,6 +19,8 @@ tensor's device and current stream, asynchronously.
 
 from __future__ import annotations
 
+import sys
+from collections.abc import Callable
 from typing import Any
 
 from .._errors import LaunchError
@@ -33,8 +35,23 @@ def _torch():
     return torch
 
 
+_PKG = sys.modules[__package__]  # hc.gfx950 (still loading here): the current device and stream
+
+
+def _on_stream(torch: Any, device: Any, launch: Callable[[int], None]) -> None:
+    """launch(raw current stream of ``device``), with that device current."""
+    if _PKG._current_device(torch) == device.index:
+        launch(_PKG._current_stream(torch, device.index))
+    else:
+        with torch.cuda.device(device):
+            launch(torch.cuda.current_stream(device).cuda_stream)
+
+
 def _origins(torch: Any, origins: Any, device: Any) -> Any:
-    o = torch.as_tensor(origins, dtype=torch.int64, device=device)
+    if isinstance(origins, torch.Tensor) and origins.dtype is torch.int64 and origins.device == device:
+        o = origins
+    else:
+        o = torch.as_tensor(origins, dtype=torch.int64, device=device)
     if o.ndim == 1 and o.numel() == 2:
         o = o.reshape(1, 2)
     if o.ndim != 2 or o.shape[1] != 2:
@@ -69,6 +86,8 @@ def _mask(torch: Any, mask: Any, shape: tuple[int, int, int], device: Any) -> An
 
 
 def _fill_bits(torch: Any, fill: Any, dtype: Any) -> int:
+    if type(fill) is int and fill == 0:
+        return 0
     v = torch.tensor([fill], dtype=dtype)
     ints = {2: torch.int16, 4: torch.int32, 8: torch.int64}[v.element_size()]
     return int(v.view(ints).item()) & ((1 << (8 * v.element_size())) - 1)
@@ -88,15 +107,14 @@ def tile_load(src: Any, origins: Any, shape: tuple[int, int], *, mask: Any = Non
     n = o.shape[0]
     m = _mask(torch, mask, (n, th, tw), src.device)
     out = torch.empty((n, th, tw), dtype=src.dtype, device=src.device)
-    active = torch.empty((n, th, tw), dtype=torch.uint8, device=src.device)
+    active = torch.empty((n, th, tw), dtype=torch.bool, device=src.device)
     if out.numel() == 0:
-        return out, active.view(torch.bool)
-    with torch.cuda.device(src.device):
-        stream = torch.cuda.current_stream(src.device).cuda_stream
-        _native.tile_load(src.element_size(), src.data_ptr(), ld, rows, cols, o.data_ptr(), n, th, tw,
-                          m.data_ptr() if m is not None else 0, _fill_bits(torch, fill, src.dtype),
-                          out.data_ptr(), active.data_ptr(), stream)
-    return out, active.view(torch.bool)
+        return out, active
+    _on_stream(torch, src.device, lambda stream: _native.tile_load(
+        src.element_size(), src.data_ptr(), ld, rows, cols, o.data_ptr(), n, th, tw,
+        m.data_ptr() if m is not None else 0, _fill_bits(torch, fill, src.dtype), out.data_ptr(), active.data_ptr(),
+        stream))
+    return out, active
 
 
 def tile_store(dst: Any, origins: Any, tiles: Any, *, mask: Any = None) -> None:
@@ -120,7 +138,6 @@ def tile_store(dst: Any, origins: Any, tiles: Any, *, mask: Any = None) -> None:
     t = tiles.contiguous()
     if t.numel() == 0 or rows == 0 or cols == 0:
         return
-    with torch.cuda.device(dst.device):
-        stream = torch.cuda.current_stream(dst.device).cuda_stream
-        _native.tile_store(dst.element_size(), dst.data_ptr(), ld, rows, cols, o.data_ptr(), n, th, tw,
-                           t.data_ptr(), m.data_ptr() if m is not None else 0, stream)
+    _on_stream(torch, dst.device, lambda stream: _native.tile_store(
+        dst.element_size(), dst.data_ptr(), ld, rows, cols, o.data_ptr(), n, th, tw, t.data_ptr(),
+        m.data_ptr() if m is not None else 0, stream))

@@ -164,12 +164,20 @@ class Const(Expr):
 class Symbol(Expr):
     """A named integer symbol (``sym.M``)."""
 
-    __slots__ = ("name",)
+    __slots__ = ("name", "_hash")
 
     def __init__(self, name: str) -> None:
         if not name or not name.isidentifier():
             raise ValueError(f"invalid symbol name {name!r}")
         self.name = name
+        self._hash = hash(("sym", name))
+
+    # (Symbols are the keys of every launch's bindings.)
+    def __hash__(self) -> int:
+        return self._hash
+
+    def __eq__(self, other: object) -> bool:
+        return True if self is other else Expr.__eq__(self, other)
 
     def eval(self, env: Mapping[Any, int] | Env) -> int:  # noqa: A003
         value = _lookup(env, self)
