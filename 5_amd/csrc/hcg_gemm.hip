@@ -1821,8 +1821,20 @@ __device__ __forceinline__ unsigned char* rs_b() {
 // with an LDS DMA in flight the compiler waits for it, and so for every
 // older load, before LDS reads.  A second block past A's last byte is
 // replaced by the first (its bytes are k >= K, cleared).
-template <int DT, int NB, bool UA = false, int ST = 0>
+//
+// WALK (by DMA, one K split, well over one row block per CU): one workgroup
+// per CU walks row blocks w, w + walkers, ... and its ring runs on from one
+// block into the next, so that a block's first loads and its stores overlap
+// the blocks beside it.  Started workgroup by workgroup, a block paid its
+// ramp-up and its end each time.  bf16/f16, us (A from HBM, three buffers in
+// turn), a workgroup per block -> walking: 65536 x 3 x 640 21.0 -> 15.4,
+// 40000 x 13 x 512 13.4 -> 10.7, 65536 x 64 x 2048 68.8 -> 61.5, 65536 x 8 x
+// 4096 103.2 -> 91.3 (5.9 TB/s; the read probe reaches 6.4), 30001 x 16 x 4001
+// 50.6 -> 48.7; with 266 blocks for 256 CUs (17000 x 33 x 8192) 98.2 -> 102.5,
+// so up to 1.25 blocks per CU keep a workgroup each.
+template <int DT, int NB, bool UA = false, int ST = 0, bool WALK = false>
 __global__ __launch_bounds__(NB == 64 ? 512 : 256) void gemm_rowstream_kernel(RowStreamArgs g) {
+  static_assert(!WALK || !UA, "walking is by DMA");
   static_assert(NB == 16 || NB == 32 || NB == 64, "column block");
   // ST = 3 (NB <= 32, register-staged A): a 72 KB ring, so two workgroups
   // share a CU -- twice the waves to cover the register path's latency
@@ -1849,8 +1861,8 @@ __global__ __launch_bounds__(NB == 64 ? 512 : 256) void gemm_rowstream_kernel(Ro
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nrb = (g.M + kRsRows - 1) / kRsRows;
-  const int split = blockIdx.x / nrb;
-  const int m0 = (blockIdx.x - split * nrb) * kRsRows;
+  const int split = WALK ? 0 : blockIdx.x / nrb;
+  const int first_rb = blockIdx.x - split * nrb;
   const int kbeg = split * g.kchunk;
   const int kend = min(g.K, kbeg + g.kchunk);
   const int nsteps = (kend - kbeg + kRsStep - 1) / kRsStep;
@@ -1869,7 +1881,8 @@ __global__ __launch_bounds__(NB == 64 ? 512 : 256) void gemm_rowstream_kernel(Ro
     const int row = kRowsPerWave * wave + 4 * i + (lane >> 4);
     const int c = (lane & 15) ^ (row & 15);
     a_col[i] = c * 8;
-    a_off[i] = UA ? 0 : ((m0 + row) * g.lda + c * 8) * 2;  // (UA reads through 64-bit pointers)
+    // (WALK: from the row block; UA reads through 64-bit pointers)
+    a_off[i] = UA ? 0 : (((WALK ? 0 : first_rb * kRsRows) + row) * g.lda + c * 8) * 2;
   }
   int b_off[kBDmaPerWave], b_row[kBDmaPerWave];
 #pragma unroll
@@ -1892,7 +1905,7 @@ __global__ __launch_bounds__(NB == 64 ? 512 : 256) void gemm_rowstream_kernel(Ro
   bool a_rowok[kAInst];
 #pragma unroll
   for (int i = 0; i < kAInst; ++i) {
-    const int row = m0 + kRowsPerWave * wave + 4 * i + (lane >> 4);
+    const int row = first_rb * kRsRows + kRowsPerWave * wave + 4 * i + (lane >> 4);
     a_rowok[i] = row < g.M;
     a_rowp[i] = a_base + (uintptr_t)(a_rowok[i] ? row : 0) * (uintptr_t)g.lda * 2;
   }
@@ -1905,13 +1918,44 @@ __global__ __launch_bounds__(NB == 64 ? 512 : 256) void gemm_rowstream_kernel(Ro
   // blocks start at 16 evenly spaced steps instead (rot_groups; 65536 x 8 x
   // 4096: 102 us, against 125 us at every step and 106 us unrotated).  Steps
   // past the run load zeros.
-  const int rg = min(g.rot_groups, nsteps);
-  const int rot = ((blockIdx.x - split * nrb) % rg) * (nsteps / rg);
-  auto issue = [&](auto sc, int step) {
+  // A walk's blocks start instead at the steps of a golden-ratio sequence
+  // (rb * 0.618.. mod 1, scaled to the steps), which spreads any run of
+  // blocks evenly: workgroups that walk drift apart less than ones dispatched
+  // as others end, and with the rule above 65536 x 8 x 4096 walks in 105.3 us
+  // against 91.3 (16384 x 8 x 16384, a block each, 93.9 against 89.5).
+  auto rot_of = [&](int rb) {
+    if constexpr (WALK)
+      return (int)(((uint64_t)((uint32_t)rb * 2654435769u) * (uint32_t)nsteps) >> 32);
+    else {
+      const int rg = min(g.rot_groups, nsteps);
+      return rb % rg * (nsteps / rg);
+    }
+  };
+  // The next stage to request, and to multiply.
+  struct Place {
+    int rb, s, rot;
+  };
+  auto advance = [&](Place& w) {
+    ++w.s;
+    if constexpr (WALK) {
+      if (w.s == nsteps) {
+        w.s = 0;
+        w.rb += gridDim.x;
+        w.rot = rot_of(w.rb);
+      }
+    }
+  };
+  auto k_of = [&](const Place& w) {
+    const int s = w.s + w.rot;
+    return kbeg + (s >= nsteps ? s - nsteps : s) * kRsStep;
+  };
+  Place to_issue{first_rb, 0, rot_of(first_rb)}, to_multiply = to_issue;
+  auto issue = [&](auto sc) {
     constexpr int S = decltype(sc)::value;
-    int s = step + rot;
-    if (s >= nsteps) s -= nsteps;
-    const int k0 = step < nsteps ? kbeg + s * kRsStep : kend;
+    const bool more = WALK ? to_issue.rb < nrb : to_issue.s < nsteps;
+    const int k0 = more ? k_of(to_issue) : kend;
+    const unsigned a_adv = ((WALK ? (unsigned)to_issue.rb * kRsRows * (unsigned)g.lda : 0u) + (unsigned)k0) * 2u;
+    advance(to_issue);
     if constexpr (UA) {
 #pragma unroll
       for (int i = 0; i < kAInst; ++i) {
@@ -1935,7 +1979,7 @@ __global__ __launch_bounds__(NB == 64 ? 512 : 256) void gemm_rowstream_kernel(Ro
 #pragma unroll
       for (int i = 0; i < kAInst; ++i)
         dma16(rsrc_a, (lds_void*)(rs_a<NB, S>() + (kRowsPerWave * wave + 4 * i) * 256),
-              dma_offset(k0 + a_col[i] < kend, a_off[i] + k0 * 2));
+              dma_offset(k0 + a_col[i] < kend, (int)((unsigned)a_off[i] + a_adv)));
 #pragma unroll
       for (int i = 0; i < kBDmaPerWave; ++i)
         dma16(rsrc_b, (lds_void*)(rs_b<NB, S>() + (wave * kBDmaPerWave + i) * 1024),
@@ -1997,12 +2041,33 @@ __global__ __launch_bounds__(NB == 64 ? 512 : 256) void gemm_rowstream_kernel(Ro
     }
   };
 
+  // The finished row block leaves.  16x16 accumulator layout: register r of
+  // lane l holds row 4*(l/16) + r, column l%16 of the block.
+  float* dst = g.splits > 1 ? g.ws + (int64_t)split * g.M * g.N : g.C;
+  const int64_t ld = g.splits > 1 ? (int64_t)g.N : g.ldc;
+  auto store = [&](int m0) {
+#pragma unroll
+    for (int cb = 0; cb < kBlocks; ++cb) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = m0 + 16 * (wave / kColSplit) + (lane >> 4) * 4 + r, col = col0 + 16 * cb + (lane & 15);
+        if (row < g.M && col < g.N) dst[(int64_t)row * ld + col] = acc[cb][r];
+      }
+      acc[cb] = f32x4{};
+    }
+  };
+
   // Same step structure as the skinny streaming kernel: wait for stage S
-  // (STAGES - 2 newer stages may be in flight), barrier, refill the
-  // stage freed one step earlier, multiply.
+  // (STAGES - 2 newer stages may be in flight; a block's stores among them
+  // only make the wait longer), barrier, refill the stage freed one step
+  // earlier, multiply.
   constexpr int kLater = STAGES - 2;
   auto step_fn = [&](auto sc, int step) {
     constexpr int S = decltype(sc)::value;
+    if constexpr (!WALK) {
+      to_multiply.s = step;
+      to_issue.s = step + STAGES - 1;
+    }
     wait_vmcnt<kLoadsPerWave * kLater>();
     if constexpr (UA) {
       // This wave's chunks of the stage have landed in registers.
@@ -2023,21 +2088,24 @@ __global__ __launch_bounds__(NB == 64 ? 512 : 256) void gemm_rowstream_kernel(Ro
     wait_lgkm0();
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    issue(StageC<(S + STAGES - 1) % STAGES>{}, step + STAGES - 1);
-    int s_k = step + rot;
-    if (s_k >= nsteps) s_k -= nsteps;
-    compute(sc, g.K - (kbeg + s_k * kRsStep));
+    issue(StageC<(S + STAGES - 1) % STAGES>{});
+    compute(sc, g.K - k_of(to_multiply));
+    const int rb = to_multiply.rb;
+    advance(to_multiply);
+    if constexpr (WALK)
+      if (to_multiply.s == 0) store(rb * kRsRows);
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  issue(StageC<0>{}, 0);
-  issue(StageC<1>{}, 1);
-  if constexpr (STAGES > 3) issue(StageC<2 % STAGES>{}, 2);
-  if constexpr (STAGES > 4) issue(StageC<3 % STAGES>{}, 3);
-  if constexpr (STAGES > 5) issue(StageC<4 % STAGES>{}, 4);
+  issue(StageC<0>{});
+  issue(StageC<1>{});
+  if constexpr (STAGES > 3) issue(StageC<2 % STAGES>{});
+  if constexpr (STAGES > 4) issue(StageC<3 % STAGES>{});
+  if constexpr (STAGES > 5) issue(StageC<4 % STAGES>{});
 
+  const int total = WALK ? (nrb - first_rb + (int)gridDim.x - 1) / (int)gridDim.x * nsteps : nsteps;
   int step = 0;
-  for (; step + STAGES <= nsteps; step += STAGES) {
+  for (; step + STAGES <= total; step += STAGES) {
     step_fn(StageC<0>{}, step);
     step_fn(StageC<1>{}, step + 1);
     step_fn(StageC<2>{}, step + 2);
@@ -2045,27 +2113,16 @@ __global__ __launch_bounds__(NB == 64 ? 512 : 256) void gemm_rowstream_kernel(Ro
     if constexpr (STAGES > 4) step_fn(StageC<4 % STAGES>{}, step + 4);
     if constexpr (STAGES > 5) step_fn(StageC<5 % STAGES>{}, step + 5);
   }
-  if (step < nsteps) step_fn(StageC<0>{}, step++);
-  if (step < nsteps) step_fn(StageC<1>{}, step++);
+  if (step < total) step_fn(StageC<0>{}, step++);
+  if (step < total) step_fn(StageC<1>{}, step++);
   if constexpr (STAGES > 3)
-    if (step < nsteps) step_fn(StageC<2 % STAGES>{}, step++);
+    if (step < total) step_fn(StageC<2 % STAGES>{}, step++);
   if constexpr (STAGES > 4)
-    if (step < nsteps) step_fn(StageC<3 % STAGES>{}, step++);
+    if (step < total) step_fn(StageC<3 % STAGES>{}, step++);
   if constexpr (STAGES > 5)
-    if (step < nsteps) step_fn(StageC<4 % STAGES>{}, step++);
+    if (step < total) step_fn(StageC<4 % STAGES>{}, step++);
   wait_vmcnt<0>();  // no DMA may still be writing LDS at exit
-
-  // 16x16 accumulator layout: register r of lane l holds row 4*(l/16) + r,
-  // column l%16 of the block.
-  float* dst = g.splits > 1 ? g.ws + (int64_t)split * g.M * g.N : g.C;
-  const int64_t ld = g.splits > 1 ? (int64_t)g.N : g.ldc;
-#pragma unroll
-  for (int cb = 0; cb < kBlocks; ++cb)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = m0 + 16 * (wave / kColSplit) + (lane >> 4) * 4 + r, col = col0 + 16 * cb + (lane & 15);
-      if (row < g.M && col < g.N) dst[(int64_t)row * ld + col] = acc[cb][r];
-    }
+  if constexpr (!WALK) store(first_rb * kRsRows);
 }
 
 // C[i][j] = sum over splits s = 0..S-1 (in order) of ws[s][i][j] (ws rows:
@@ -2906,7 +2963,7 @@ bool rowstream_fits(const void* A, int64_t lda, const void* B, int64_t ldb, int6
 }
 
 template <int DT, int NB>
-void launch_rowstream(const RowStreamArgs& a, bool ua, bool short_ring, dim3 grid, hipStream_t stream) {
+void launch_rowstream(const RowStreamArgs& a, bool ua, bool short_ring, bool walk, dim3 grid, hipStream_t stream) {
   if constexpr (NB <= 32) {
     if (short_ring) {
       if (ua)
@@ -2917,7 +2974,9 @@ void launch_rowstream(const RowStreamArgs& a, bool ua, bool short_ring, dim3 gri
     }
   }
   const dim3 block(NB == 64 ? 512 : 256);
-  if (ua)
+  if (walk)
+    gemm_rowstream_kernel<DT, NB, false, 0, true><<<grid, block, 0, stream>>>(a);
+  else if (ua)
     gemm_rowstream_kernel<DT, NB, true><<<grid, block, 0, stream>>>(a);
   else
     gemm_rowstream_kernel<DT, NB, false><<<grid, block, 0, stream>>>(a);
@@ -2981,16 +3040,19 @@ int run_rowstream(const Scratch& sc, int dtype, const void* A, int64_t lda, cons
   // Extents end with the chunk that holds the last element.
   a.a_bytes = a_dma ? (int)((((int64_t)M - 1) * lda + (int64_t)round_up(K, 8)) * 2) : 0;
   a.b_bytes = (int)((((int64_t)K - 1) * a.ldb + (int64_t)round_up(N, 8)) * 2);
-  const dim3 grid((unsigned)(nrb * a.splits));
+  // One workgroup per CU (the ring takes a CU's LDS) walks the row blocks when
+  // there are over 1.25 per CU (see WALK).
+  const bool walk = a.splits == 1 && a_dma && (int64_t)4 * nrb >= (int64_t)5 * st->num_cus;
+  const dim3 grid((unsigned)(walk ? st->num_cus : nrb * a.splits));
   const int nb = N <= 16 ? 16 : N <= 32 ? 32 : 64;
   if (dtype == HCG_F16) {
-    if (nb == 16) launch_rowstream<HCG_F16, 16>(a, !a_dma, short_ring, grid, stream);
-    else if (nb == 32) launch_rowstream<HCG_F16, 32>(a, !a_dma, short_ring, grid, stream);
-    else launch_rowstream<HCG_F16, 64>(a, !a_dma, short_ring, grid, stream);
+    if (nb == 16) launch_rowstream<HCG_F16, 16>(a, !a_dma, short_ring, walk, grid, stream);
+    else if (nb == 32) launch_rowstream<HCG_F16, 32>(a, !a_dma, short_ring, walk, grid, stream);
+    else launch_rowstream<HCG_F16, 64>(a, !a_dma, short_ring, walk, grid, stream);
   } else {
-    if (nb == 16) launch_rowstream<HCG_BF16, 16>(a, !a_dma, short_ring, grid, stream);
-    else if (nb == 32) launch_rowstream<HCG_BF16, 32>(a, !a_dma, short_ring, grid, stream);
-    else launch_rowstream<HCG_BF16, 64>(a, !a_dma, short_ring, grid, stream);
+    if (nb == 16) launch_rowstream<HCG_BF16, 16>(a, !a_dma, short_ring, walk, grid, stream);
+    else if (nb == 32) launch_rowstream<HCG_BF16, 32>(a, !a_dma, short_ring, walk, grid, stream);
+    else launch_rowstream<HCG_BF16, 64>(a, !a_dma, short_ring, walk, grid, stream);
   }
   HCG_HIP_CHECK(hipGetLastError());
   if (a.splits > 1) return launch_reduce(a.ws, C, ldc, M, N, M, a.splits, aligned16(C) && ldc % 4 == 0, stream);

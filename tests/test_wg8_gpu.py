@@ -141,3 +141,14 @@ def test_transposed_operand_under_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
+
+
+# Over 1.25 row blocks of 64 per CU the narrow kernel walks several blocks per
+# workgroup: a block's last stage beside the next one's first, K of one stage
+# (so that every stage ends a block), below one and ragged, the last block
+# ragged, workgroups with one block more than others.
+@pytest.mark.parametrize("m,n,k", [(20481, 8, 128), (20417, 1, 1), (33000, 16, 130), (40963, 17, 500), (24000, 33, 1001),
+                                   (32768, 64, 640), (50001, 40, 257)])
+@pytest.mark.parametrize("dtype", list(DTYPES))
+def test_narrow_kernel_walks_row_blocks(m, n, k, dtype):
+    _check(m, n, k, dtype, 3 if dtype == "float16" else 8)
