@@ -28,9 +28,9 @@
 //     LDS once by DMA, split over K across workgroups mapped so every XCD
 //     covers all column residues, against 1, 2, 4 or 8 16-row blocks of A;
 //     the split partials are summed in a fixed order (deterministic) by
-//     the last workgroup of each column block to arrive (R <= 2) or by
-//     stream_reduce_kernel, skinny_reduce_kernel or, past 16 splits,
-//     split_reduce_kernel.  Its UB form stages B through registers when
+//     the last workgroup of each column block to arrive (where they are
+//     small) or by stream_reduce_kernel, skinny_reduce_kernel or, past 16
+//     splits, split_reduce_kernel.  Its UB form stages B through registers when
 //     B's last row piece cannot be read safely in place.
 //   * gemm_generic_kernel -- fallback (plain pointers, register staging, any
 //     alignment) for unaligned operands whose byte offsets do not fit 31
@@ -65,6 +65,7 @@
 
 #include "hcg_gemm.h"
 #include "hcg_runtime.h"
+#include "hcg_splitsum.h"
 #include "hcg_tile.h"
 
 namespace hcg {
@@ -1217,15 +1218,12 @@ __global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(SkinnyArgs 
 // feeds R MFMAs.  Each block's 16x32 slice of a stage arrives by one more
 // DMA instruction (block rb from wave rb % 4).
 //
-// Split-K partials go to a workspace [splits][16 R][N].  With at most
-// kStFuseMaxSplits(R) splits, R <= 2 and N a multiple of 4 the workgroups of a
-// column block reduce them themselves: each publishes its partial with
-// agent-scope (L2-coherent across XCDs) stores and counts its arrival on the
-// column block's counter; the last to arrive sums the partials in order
-// s = 0..S-1, writes C and resets the counter.  Otherwise (and for the
-// allocation-free entry point, which has no counters) stream_reduce_kernel
-// sums them in a second launch, in the same order: results are bit-identical
-// either way.
+// Split-K partials go to a workspace.  Where they are small (R <= 4,
+// kMaxSummedBytes) the last workgroup of a column block to arrive sums them in
+// order s = 0..S-1 and writes C (sum_splits, hcg_splitsum.h).  Otherwise (and
+// for the allocation-free entry point, which has no counters) they are rows
+// [splits][16 R][N] that stream_reduce_kernel sums in a second launch, in the
+// same order: results are bit-identical either way.
 
 constexpr int kStN = 128;
 constexpr int kStStep = 32;
@@ -1234,13 +1232,10 @@ constexpr int kStBBytes = kStStep * kStN * 2;  // 8 KB
 constexpr int kStABytes = 16 * kStStep * 2;    // 1 KB per 16-row block of A
 constexpr int kStMaxRowBlocks = 8;              // M <= 128
 constexpr int kStMaxSplits = 16;      // partials stream_reduce_kernel holds in registers
-// Splits the in-kernel reduction takes with R row blocks (its registers
-// hold every other split's partial; more would cost the kernel occupancy).
-constexpr int kStFuseMaxSplits(int R) { return R == 1 ? 8 : 4; }
-constexpr int kStCounterBytes = 16384;  // arrival counters ahead of each workspace: 4096 column blocks
-// Cache policy of a buffer access coherent at agent scope on gfx950 (SC1):
-// the bits the compiler gives a relaxed agent-scope atomic load or store.
-constexpr int kCpolAgent = 16;
+// Row blocks up to which the last workgroup of a column block sums its K
+// splits (hcg_splitsum.h); R = 8's partials are 64 KB each.
+constexpr bool stream_can_fuse(int R) { return R <= 4; }
+constexpr int kStCounterBytes = 16384;  // arrival counters ahead of each workspace: 256 of them, 64 bytes apart
 constexpr int kStMaxSplitsLoop = 256;  // K splits at all (more than 16: split_reduce_kernel)
 
 struct StreamArgs {
@@ -1256,7 +1251,7 @@ struct StreamArgs {
   int rblocks;    // 16-row blocks of A: 1, 2, 4 or 8 (M <= 16 * rblocks)
   int a_bytes, b_bytes;
   bool c_vec;     // C rows 16-byte aligned at every 4th column
-  unsigned* counters;  // per column block arrival counters (all zero between launches), or null
+  unsigned* counters;  // per column block arrival counters (sum_splits), or null
   int ws_bytes;        // bytes of the partials (with counters: below 2^31)
 #ifdef HCG_STAMPS
   int stamp_slot;
@@ -1329,98 +1324,6 @@ __device__ __forceinline__ unsigned char* st_a() {
 // stored at c ^ ((r >> 2) & 3), so the 16 rows read at one chunk hit 16
 // distinct 16-byte bank groups.
 __device__ __forceinline__ int sta_swz(int row, int c) { return c ^ ((row >> 2) & 3); }
-
-// The split-K reduction inside the streaming kernel (R <= 2 row blocks,
-// N % 4 == 0, splits <= kStFuseMaxSplits(R); the host checks).  Called by every
-// thread of the workgroup of (column block nb, split) after its K loop,
-// with the wave's 16x16 accumulators (register r of lane l: row 4 (l/16) + r,
-// column l%16 of the wave's column block j).
-template <int R>
-__device__ __forceinline__ void stream_fused_reduce(const StreamArgs& g, const f32x4 (&acc)[R][kStN / 64],
-                                                    int nb, int split) {
-  constexpr int NB = kStN;
-  constexpr int kColsPerWave = NB / 4;
-  constexpr int kBlocks = kColsPerWave / 16;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int n0 = nb * NB;
-  // The arrival count is broadcast through B stage 7 (free after the K loop;
-  // a separate LDS variable would push two R = 2 workgroups past the CU's
-  // 160 KB).
-  unsigned* s_arrived = reinterpret_cast<unsigned*>(st_b<kStStages - 1>());
-  // Stage the 16R x 128 partial through LDS (row block rb in B stage rb:
-  // 16 x 128 floats = 8 KB), so that each thread then holds two whole
-  // 16-byte row pieces.  Every wave has finished reading the stages.
-  __syncthreads();
-#pragma unroll
-  for (int rb = 0; rb < R; ++rb) {
-    float* ep = reinterpret_cast<float*>(rb == 0 ? st_b<0>() : st_b<1>());
-#pragma unroll
-    for (int j = 0; j < kBlocks; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        ep[((lane >> 4) * 4 + r) * NB + wave * kColsPerWave + 16 * j + (lane & 15)] = acc[rb][j][r];
-  }
-  __syncthreads();
-  // Piece c (of 512 per row block): row c / 32, columns 4 (c % 32) .. +3.
-  // N % 4 == 0, so a piece is either wholly inside N or wholly past it.
-  const __amdgpu_buffer_rsrc_t rws = make_rsrc(g.ws, g.ws_bytes);
-  u32x4 mine[R][2];
-#pragma unroll
-  for (int rb = 0; rb < R; ++rb)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int c = tid + 256 * h, row = c >> 5, col = n0 + (c & 31) * 4;
-      const float* ep = reinterpret_cast<const float*>(rb == 0 ? st_b<0>() : st_b<1>());
-      mine[rb][h] = *reinterpret_cast<const u32x4*>(ep + row * NB + (c & 31) * 4);
-      if (col < g.N)
-        __builtin_amdgcn_raw_buffer_store_b128(mine[rb][h], rws,
-                                               (int)((((int64_t)split * 16 * R + 16 * rb + row) * g.N + col) * 4), 0,
-                                               kCpolAgent);
-    }
-  // The partial is visible at agent scope once its stores have completed;
-  // only then is the arrival counted.
-  wait_vmcnt<0>();
-  __syncthreads();
-  if (tid == 0) *s_arrived = __hip_atomic_fetch_add(g.counters + nb, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __syncthreads();
-  if (*s_arrived != (unsigned)(g.splits - 1)) return;
-  // Last arrival: every other split's partial is complete.  The counter is
-  // reset for the next launch (which follows this one in stream order).
-  if (tid == 0) __hip_atomic_store(g.counters + nb, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  constexpr int kMaxSplits = kStFuseMaxSplits(R);
-  u32x4 part[kMaxSplits][R][2];
-#pragma unroll
-  for (int sp = 0; sp < kMaxSplits; ++sp)
-#pragma unroll
-    for (int rb = 0; rb < R; ++rb)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int c = tid + 256 * h, row = c >> 5, col = n0 + (c & 31) * 4;
-        part[sp][rb][h] = u32x4{0, 0, 0, 0};
-        if (sp < g.splits && sp != split && col < g.N)
-          part[sp][rb][h] = __builtin_amdgcn_raw_buffer_load_b128(
-              rws, (int)((((int64_t)sp * 16 * R + 16 * rb + row) * g.N + col) * 4), 0, kCpolAgent);
-      }
-  // Sum in split order, as stream_reduce_kernel does.
-#pragma unroll
-  for (int rb = 0; rb < R; ++rb)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int c = tid + 256 * h, row = 16 * rb + (c >> 5), col = n0 + (c & 31) * 4;
-      if (row >= g.M || col >= g.N) continue;
-      f32x4 v = __builtin_bit_cast(f32x4, split == 0 ? mine[rb][h] : part[0][rb][h]);
-#pragma unroll
-      for (int sp = 1; sp < kMaxSplits; ++sp)
-        if (sp < g.splits) v += __builtin_bit_cast(f32x4, sp == split ? mine[rb][h] : part[sp][rb][h]);
-      float* dst = g.C + (int64_t)row * g.ldc + col;
-      if (g.c_vec) {
-        *reinterpret_cast<f32x4*>(dst) = v;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) dst[e] = v[e];
-      }
-    }
-}
 
 // UB (B's last row piece not safely readable in place, so no DMA for B):
 // each lane fetches the two aligned 16-byte blocks around its B chunk PF
@@ -1684,7 +1587,19 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(StreamArgs g) {
   // 16x16 accumulator layout: register r of lane l holds row 4*(l/16) + r,
   // column l%16 of the block.
   const int ocol = n0 + wave * kColsPerWave + (lane & 15);
-  if (g.splits == 1) {
+  bool to_c = g.splits == 1;
+  if constexpr (stream_can_fuse(R)) {
+    if (!to_c && g.counters != nullptr) {
+      to_c = hcg::sum_splits<R * kBlocks, 256>(reinterpret_cast<f32x4(&)[R * kBlocks]>(acc),
+                                               make_rsrc(g.ws, g.ws_bytes), (g.N + NB - 1) / NB, nb, g.splits, split,
+                                               g.counters, reinterpret_cast<unsigned*>(st_b<0>()));
+      if (!to_c) {
+        stamps.write();
+        return;
+      }
+    }
+  }
+  if (to_c) {
 #pragma unroll
     for (int rb = 0; rb < R; ++rb)
 #pragma unroll
@@ -1696,13 +1611,6 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(StreamArgs g) {
         }
     stamps.write();
     return;
-  }
-  if constexpr (R <= 2) {
-    if (g.counters != nullptr) {
-      stream_fused_reduce<R>(g, acc, nb, split);
-      stamps.write();
-      return;
-    }
   }
 #pragma unroll
   for (int rb = 0; rb < R; ++rb)
@@ -1755,6 +1663,8 @@ struct RowStreamArgs {
   int kchunk;     // K per split, multiple of kRsStep
   int splits;
   int a_bytes, b_bytes;
+  unsigned* counters;  // per row block, or null: a second launch sums the partials
+  int ws_bytes;        // (with counters) bytes of the partials
   int rot_groups;  // distinct start steps over the row blocks (>= the run's steps: every step)
 };
 
@@ -2043,8 +1953,9 @@ __global__ __launch_bounds__(NB == 64 ? 512 : 256) void gemm_rowstream_kernel(Ro
 
   // The finished row block leaves.  16x16 accumulator layout: register r of
   // lane l holds row 4*(l/16) + r, column l%16 of the block.
-  float* dst = g.splits > 1 ? g.ws + (int64_t)split * g.M * g.N : g.C;
-  const int64_t ld = g.splits > 1 ? (int64_t)g.N : g.ldc;
+  const bool to_ws = g.splits > 1 && g.counters == nullptr;
+  float* dst = to_ws ? g.ws + (int64_t)split * g.M * g.N : g.C;
+  const int64_t ld = to_ws ? (int64_t)g.N : g.ldc;
   auto store = [&](int m0) {
 #pragma unroll
     for (int cb = 0; cb < kBlocks; ++cb) {
@@ -2122,7 +2033,13 @@ __global__ __launch_bounds__(NB == 64 ? 512 : 256) void gemm_rowstream_kernel(Ro
   if constexpr (STAGES > 5)
     if (step < total) step_fn(StageC<4 % STAGES>{}, step++);
   wait_vmcnt<0>();  // no DMA may still be writing LDS at exit
-  if constexpr (!WALK) store(first_rb * kRsRows);
+  if constexpr (!WALK) {
+    if (g.splits > 1 && g.counters != nullptr &&
+        !hcg::sum_splits<kBlocks, 64 * kWaves>(acc, make_rsrc(g.ws, g.ws_bytes), nrb, first_rb, g.splits, split,
+                                               g.counters, reinterpret_cast<unsigned*>(rs_a<NB, 0>())))
+      return;
+    store(first_rb * kRsRows);
+  }
 }
 
 // C[i][j] = sum over splits s = 0..S-1 (in order) of ws[s][i][j] (ws rows:
@@ -2556,7 +2473,8 @@ constexpr double kLaunchUs = 2.0;
 // plus the traffic, and 2.5 us of host time, so that small calls take at
 // least 6.6 us.  Both sides, us: 128 x 8192 x 8192 (4 parts of 64 KB) 34.4
 // fused, 35.8 not; 1024 x 1024 x 4096 14.7 / 16.3; 192 x 192 x 1440 5.7 /
-// 6.8; 512 x 512 x 16384 in 16 parts 26.4 / 15.8.
+// 6.8; 512 x 512 x 16384 in 8 parts of 32 KB fused 17.5 to 18.9 over five
+// boxes, in 16 parts 24.6 to 26.4 fused and 15.8 to 24.3 not.
 struct TilePlan {
   int shape;
   int splits;
@@ -2587,7 +2505,7 @@ bool fused_ok(const TileShape& t, int splits, int M, int N, int K, size_t room) 
   const size_t limit = room < kMaxSplitWorkspace ? room : kMaxSplitWorkspace;
   return t.wg8 && hcg::wg8::can_fuse(t.tm, t.tn) && splits > 1 && splits <= 16 &&
          (K + splits - 1) / splits >= kMinKPerFusedSplit &&
-         plan_tile_count(t, M, N) * hcg::wg8::kCounterStride * 4 <= kStCounterBytes &&
+         plan_tile_count(t, M, N) * hcg::kSplitCounterStride * 4 <= kStCounterBytes &&
          fused_bytes(t, splits, M, N) <= limit;
 }
 
@@ -2603,7 +2521,7 @@ double plan_cost(const TileShape& t, int splits, bool fused, int num_cus, int M,
     if (fused) {
       us += 1.0 + (splits - 1) * (t.tm * t.tn * 4) / 1.0e5 + (double)fused_bytes(t, splits, M, N) / 3.0e6;
     } else {
-      us += 4.2 + (double)(splits + 1) * M * N * sizeof(float) / 4.5e6;
+      us += 5.0 + (double)(splits + 1) * M * N * sizeof(float) / 4.5e6;
       if (us < 6.6) us = 6.6;
     }
   }
@@ -2629,7 +2547,8 @@ TilePlan plan_tiles(int num_cus, int M, int N, int K, int force_shape, bool allo
     if (plan_tile_count(t, M, N) * 64 > 0x7fffffff) continue;
     for (int c = 0; c < (forced_splits > 0 ? 1 : (int)(sizeof(kSplitCandidates) / sizeof(int))); ++c) {
       const int splits = forced_splits > 0 ? forced_splits : kSplitCandidates[c];
-      if (splits > 1 && !allow_split) break;
+      // (candidates ascend: once a part is too short for either form, so are the rest)
+      if (splits > 1 && (!allow_split || (K + splits - 1) / splits < kMinKPerFusedSplit)) break;
       for (int f = 0; f < 2; ++f) {
         if (f ? !(fuse && fused_ok(t, splits, M, N, K, room)) : !split_ok(splits, M, N, K, room)) continue;
         const double cost = plan_cost(t, splits, f != 0, num_cus, M, N, K);
@@ -2876,11 +2795,15 @@ int run_skinny(const Scratch& sc, int dtype, const void* A, int64_t lda, const v
     a.counters = nullptr;
     // Workspace: A repacked (when it cannot be used in place), then the
     // split partials.
-    const size_t p_sz = a.splits > 1 ? (size_t)a.splits * 16 * a.rblocks * (size_t)N * sizeof(float) : 0;
-    // The in-kernel reduction (see stream_fused_reduce) replaces the reduce
-    // launch: 16 x 8192 x 8192 fp16 25.9-26.0 -> 25.6-25.7 us.
-    const bool fuse = a.splits > 1 && a.rblocks <= 2 && a.splits <= kStFuseMaxSplits(a.rblocks) && N % 4 == 0 &&
-                      (N + kStN - 1) / kStN <= kStCounterBytes / 4 && p_sz < ((size_t)1 << 31);
+    // Whole column blocks when the last workgroup sums them; else rows of N.
+    const int nblocks = (N + kStN - 1) / kStN;
+    const size_t fused_sz = (size_t)a.splits * 16 * a.rblocks * nblocks * kStN * sizeof(float);
+    const bool fuse = !sc.fixed && a.splits > 1 && stream_can_fuse(a.rblocks) && a.splits <= hcg::kMaxSummedSplits &&
+                      a.splits * 16 * a.rblocks * kStN * 4 <= hcg::kMaxSummedBytes &&
+                      nblocks * hcg::kSplitCounterStride * 4 <= kStCounterBytes && fused_sz < ((size_t)1 << 31);
+    const size_t p_sz = fuse           ? fused_sz
+                        : a.splits > 1 ? (size_t)a.splits * 16 * a.rblocks * (size_t)N * sizeof(float)
+                                       : 0;
     if (a_sz + p_sz > 0) {
       void* ws = nullptr;
       unsigned* counters = nullptr;
@@ -3020,11 +2943,18 @@ int run_rowstream(const Scratch& sc, int dtype, const void* A, int64_t lda, cons
   a.kchunk = (ksteps + splits - 1) / splits * kRsStep;
   a.rot_groups = lda == 4096 ? 16 : 0x7fffffff;  // measured: 8 KB rows prefer 16 start steps
   a.splits = (K + a.kchunk - 1) / a.kchunk;
-  const size_t p_sz = a.splits > 1 ? (size_t)a.splits * M * N * sizeof(float) : 0;
+  // With small partials the last workgroup of a row block sums them.
+  const int nb = N <= 16 ? 16 : N <= 32 ? 32 : 64;
+  const size_t fused_sz = (size_t)a.splits * nrb * kRsRows * nb * sizeof(float);
+  const bool fuse = !sc.fixed && a.splits > 1 && a.splits <= hcg::kMaxSummedSplits &&
+                    a.splits * kRsRows * nb * 4 <= hcg::kMaxSummedBytes &&
+                    nrb * hcg::kSplitCounterStride * 4 <= kStCounterBytes && fused_sz < ((size_t)1 << 31);
+  const size_t p_sz = fuse ? fused_sz : a.splits > 1 ? (size_t)a.splits * M * N * sizeof(float) : 0;
   if (b_sz + p_sz > 0) {
     void* ws = nullptr;
-    const int rc = get_scratch(sc, b_sz + p_sz, &ws);
+    const int rc = get_scratch(sc, b_sz + p_sz, &ws, fuse ? &a.counters : nullptr);
     if (rc != HCG_OK) return rc;
+    a.ws_bytes = fuse ? (int)p_sz : 0;
     if (!b_ok) {
       uint16_t* b_p = static_cast<uint16_t*>(ws);
       const RepackJob ja{};
@@ -3044,7 +2974,6 @@ int run_rowstream(const Scratch& sc, int dtype, const void* A, int64_t lda, cons
   // there are over 1.25 per CU (see WALK).
   const bool walk = a.splits == 1 && a_dma && (int64_t)4 * nrb >= (int64_t)5 * st->num_cus;
   const dim3 grid((unsigned)(walk ? st->num_cus : nrb * a.splits));
-  const int nb = N <= 16 ? 16 : N <= 32 ? 32 : 64;
   if (dtype == HCG_F16) {
     if (nb == 16) launch_rowstream<HCG_F16, 16>(a, !a_dma, short_ring, walk, grid, stream);
     else if (nb == 32) launch_rowstream<HCG_F16, 32>(a, !a_dma, short_ring, walk, grid, stream);
@@ -3055,7 +2984,8 @@ int run_rowstream(const Scratch& sc, int dtype, const void* A, int64_t lda, cons
     else launch_rowstream<HCG_BF16, 64>(a, !a_dma, short_ring, walk, grid, stream);
   }
   HCG_HIP_CHECK(hipGetLastError());
-  if (a.splits > 1) return launch_reduce(a.ws, C, ldc, M, N, M, a.splits, aligned16(C) && ldc % 4 == 0, stream);
+  if (a.splits > 1 && a.counters == nullptr)
+    return launch_reduce(a.ws, C, ldc, M, N, M, a.splits, aligned16(C) && ldc % 4 == 0, stream);
   return HCG_OK;
 }
 
@@ -3305,8 +3235,9 @@ double stream_us(double bytes) { return 8.0 + bytes / 5.0e6; }
 Peel plan_peel(const DeviceState* st, const void* A, int64_t lda, const void* B, int64_t ldb, int M, int N,
                int K) {
   Peel p;
-  double best = 0.95 * tiled_cost(st->num_cus, M, N, K);  // a clear gain pays for the second launch
   const int rm = M % 256;
+  if (!(M > 256 && rm > 0 && rm <= 128) && !(N > 256 && N % 256 > 0 && N % 256 <= 64)) return p;
+  double best = 0.95 * tiled_cost(st->num_cus, M, N, K);  // a clear gain pays for the second launch
   if (M > 256 && rm > 0 && rm <= 128 &&
       (rm <= 16 || stream_fits(static_cast<const uint16_t*>(A) + (int64_t)(M - rm) * lda, lda, B, ldb, rm, N, K))) {
     const double c = tiled_cost(st->num_cus, M - rm, N, K) +

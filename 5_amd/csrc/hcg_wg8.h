@@ -29,6 +29,7 @@
 #include <stdint.h>
 
 #include "hcg_gemm.h"
+#include "hcg_splitsum.h"
 #include "hcg_tile.h"
 
 namespace hcg {
@@ -43,12 +44,6 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 512;
 constexpr int kWaves = 8;
-// Arrival counters (32-bit) lie 64 bytes apart, so that the tiles' atomics do
-// not queue on one line (512 x 512 x 16384 in 8 splits: 19.4 -> 18.6 us).
-constexpr int kCounterStride = 16;
-// Cache policy of an agent-scope buffer access (SC1).
-constexpr int kCpolAgent = 16;
-
 struct Args {
   const uint16_t* A;
   const uint16_t* B;
@@ -75,8 +70,9 @@ struct Args {
 #endif
 };
 
-// Tiles whose split partials the workgroups sum themselves: a thread holds
-// its own pieces and a batch of others' in registers (128x256 would spill).
+// Tiles whose split partials the workgroups sum themselves (hcg_splitsum.h): a
+// thread holds its own pieces and a batch of others' in registers (128x256
+// would spill).
 constexpr bool can_fuse(int tm, int tn) { return tm * tn <= 128 * 128; }
 
 template <int N>
@@ -478,11 +474,6 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wg8_kernel(Args g) {
       }
     }
   };
-  // A partial's piece p of thread t lies at byte 16 (512 p + t) of the (split,
-  // tile) slice: writer and reader are the same thread index.
-  const __amdgpu_buffer_rsrc_t rws = make_rsrc(g.ws, g.ws_bytes);
-  const int ntiles = g.tiles_m * g.tiles_n, tile = tm * g.tiles_n + tn;
-  auto slice = [&](int sp) { return (sp * ntiles + tile) * (TM * TN * 4) + tid * 16; };
   f32x4 mine[kMine];
   auto ep_block = [&](auto ic) {
     constexpr int I = decltype(ic)::value;
@@ -516,12 +507,6 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wg8_kernel(Args g) {
     if (!fused) {
 #pragma unroll
       for (int p = 0; p < kPieces; ++p) store_piece(mine[I * kPieces + p], I * kPieces + p);
-    } else {
-      // Agent-scope (written through to the point that all XCDs' L2s share).
-#pragma unroll
-      for (int p = 0; p < kPieces; ++p)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, mine[I * kPieces + p]), rws,
-                                               slice(split) + (I * kPieces + p) * kThreads * 16, 0, kCpolAgent);
     }
   };
   ep_block(StageC<0>{});
@@ -539,50 +524,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wg8_kernel(Args g) {
     ep_block(StageC<7>{});
   }
   if constexpr (can_fuse(TM, TN)) {
-    if (!fused) {
-      stamps.write();
-      return;
+    if (fused && sum_splits<kMine, kThreads>(mine, make_rsrc(g.ws, g.ws_bytes), g.tiles_m * g.tiles_n,
+                                             tm * g.tiles_n + tn, g.splits, split, g.counters,
+                                             reinterpret_cast<unsigned*>(ring_stage<kStageBytes, STAGES - 1>()))) {
+#pragma unroll
+      for (int p = 0; p < kMine; ++p) store_piece(mine[p], p);
     }
-    // The partial is visible at agent scope once its stores have completed;
-    // only then is the arrival counted.  The tile's last workgroup to arrive
-    // sums all partials in the order of their split and writes C; it waits
-    // for nobody, so any number of workgroups may be resident.
-    unsigned* arrived = reinterpret_cast<unsigned*>(ring_stage<kStageBytes, STAGES - 1>());
-    wait_vm<0>();
-    __syncthreads();
-    if (tid == 0)
-      *arrived = __hip_atomic_fetch_add(g.counters + tile * kCounterStride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (*arrived != (unsigned)(g.splits - 1)) {
-      stamps.write();
-      return;
-    }
-    if (tid == 0) __hip_atomic_store(g.counters + tile * kCounterStride, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // kBatch splits' loads in flight at a time: 32 of 16 bytes a thread, 16
-    // for 64x64 tiles, whose two workgroups per CU leave 128 registers.
-    constexpr int kBatch = kMine <= 2 ? 8 : 32 / kMine;
-    f32x4 sum[kMine];
-    for (int s0 = 0; s0 < g.splits; s0 += kBatch) {
-      u32x4 part[kBatch][kMine];
-#pragma unroll
-      for (int q = 0; q < kBatch; ++q)
-        if (s0 + q < g.splits && s0 + q != split) {
-#pragma unroll
-          for (int p = 0; p < kMine; ++p)
-            part[q][p] = __builtin_amdgcn_raw_buffer_load_b128(rws, slice(s0 + q) + p * kThreads * 16, 0, kCpolAgent);
-        }
-#pragma unroll
-      for (int q = 0; q < kBatch; ++q)
-        if (s0 + q < g.splits) {
-#pragma unroll
-          for (int p = 0; p < kMine; ++p) {
-            const f32x4 v = s0 + q == split ? mine[p] : __builtin_bit_cast(f32x4, part[q][p]);
-            sum[p] = s0 + q == 0 ? v : sum[p] + v;
-          }
-        }
-    }
-#pragma unroll
-    for (int p = 0; p < kMine; ++p) store_piece(sum[p], p);
   }
   stamps.write();
 }

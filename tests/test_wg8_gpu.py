@@ -152,3 +152,31 @@ def test_transposed_operand_under_capture():
 @pytest.mark.parametrize("dtype", list(DTYPES))
 def test_narrow_kernel_walks_row_blocks(m, n, k, dtype):
     _check(m, n, k, dtype, 3 if dtype == "float16" else 8)
+
+
+# K splits summed by a block's last workgroup against the same partials summed
+# by a second launch, which hcg_gemm_noalloc keeps: in the same order, so bit
+# for bit, with new operands every round (a stale partial would show).  The
+# streaming kernel with N not a multiple of 4, of 128 and with four row blocks;
+# the narrow kernel with 16, 32 and 64 columns.
+@pytest.mark.parametrize("m,n,k", [(16, 8191, 8192), (1, 1001, 4096), (31, 4099, 2048), (64, 8192, 8192),
+                                   (40, 3001, 8191), (4096, 13, 8192), (2048, 24, 12000), (4096, 64, 1024),
+                                   (300, 5, 900), (1000, 33, 4001)])
+def test_summed_splits_match_the_reduce_launch(m, n, k):
+    from hc.gfx950 import _native
+
+    print(f"case summed splits m={m} n={n} k={k}", flush=True)
+    lib = _native.load()
+    stream = torch.cuda.current_stream().cuda_stream
+    for rnd in range(4):
+        gen = torch.Generator(device=DEV).manual_seed(rnd)
+        a = torch.randn((m, k), generator=gen, device=DEV).half()
+        b = torch.randn((k, n), generator=gen, device=DEV).half()
+        outs = []
+        for entry in (lib.hcg_gemm, lib.hcg_gemm_noalloc):
+            c = torch.full((m, n), float("nan"), dtype=torch.float32, device=DEV)
+            rc = entry(_native.HCG_F16, a.data_ptr(), k, b.data_ptr(), n, c.data_ptr(), n, m, n, k, stream)
+            assert rc == _native.HCG_OK, _native.last_error(lib)
+            outs.append(c)
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0], outs[1]), rnd
