@@ -3072,8 +3072,16 @@ int run_tiled(const Scratch& sc, int dtype, const void* A, int64_t lda, const vo
   const size_t a_sz = a_ok ? 0 : round_up((size_t)M * lda_p * 2, 256);
   const size_t b_sz = b_ok ? 0 : round_up((size_t)K * ldb_p * 2, 256);
   // Explicit tile shapes run without a K split; "auto" and "tiled" may split.
-  const TilePlan plan = plan_tiles(st->num_cus, M, N, K, force_shape, force_shape < 0, nullptr,
-                                   sc.room(a_sz + b_sz), kRowMajor, sc.fixed == nullptr);
+  const size_t room = sc.room(a_sz + b_sz);
+  TilePlan plan = plan_tiles(st->num_cus, M, N, K, force_shape, force_shape < 0, nullptr, room);
+  if (plan.fused && sc.fixed) {
+    // The fixed buffer has no counters: the same splits by a second launch
+    // (the same sums in the same order) where their partials fit.
+    if ((size_t)plan.splits * M * N * sizeof(float) <= room)
+      plan.fused = false;
+    else
+      plan = plan_tiles(st->num_cus, M, N, K, force_shape, force_shape < 0, nullptr, room, kRowMajor, false);
+  }
   const TileShape& ts = kTileShapes[plan.shape];
   if ((int64_t)((M + ts.tm - 1) / ts.tm) * ((N + ts.tn - 1) / ts.tn) * plan.splits > 0x7fffffff)
     return run_generic(dtype, A, lda, B, ldb, C, ldc, M, N, K, stream);
@@ -3305,22 +3313,29 @@ int gemm_impl(int algo, int dtype, const void* A, int64_t lda, const void* B, in
 
   // N <= 64 is HBM-bound on A: stream A in 256-byte row pieces (for M <=
   // 128 too -- 64 x 32 x 2^20 fp16: 36 us against 154 us on the skinny
-  // kernel, which streams B in 128-column blocks mostly past N).
+  // kernel, which streams B in 128-column blocks mostly past N).  M <= 64 is
+  // HBM-bound on B, streamed by the skinny kernel.  But where the large
+  // operand fits the Infinity Cache several times over (64 MiB) and K is no
+  // longer than a tile plan can split, the small tiles of the tiled kernel
+  // are ahead of both from 17 rows or 33 columns on: fp16 us, three buffers
+  // in turn, streaming -> tiled: 17 x 4000 x 1024 7.2 -> 5.6, 17 x 700 x 8000
+  // 9.0 / 10.2, 33 x 700 x 8000 10.5 / 10.4, 33 x 4000 x 4096 12.9 -> 10.0,
+  // 64 x 1000 x 1000 8.5 -> 6.1, 64 x 8192 x 4096 (64 MiB) 17.7 -> 15.3, 64 x 8192 x 8192 30.4 / 32.1;
+  // 2048 x 33 x 512 6.3 -> 4.8, 4096 x 64 x 8192 17.9 -> 14.0, 8192 x 64 x 8192
+  // 31.9 / 33.4.  With 17 to 32 columns they are even (4000 x 17 x 2000 8.6 /
+  // 9.2), and 16 rows (16 x 4000 x 2000 8.2 / 8.9) or fewer stream.  Rows
+  // 65 .. 128 go to the tiled kernel whatever B's size.  It needs the large
+  // operand readable in place.
+  const int64_t kCached = (int64_t)64 << 20;
+  const auto in_place = [](const void* p, int64_t rows, int64_t cols, int64_t ld, bool whole) {
+    return (whole && aligned16(p) && ld % 8 == 0) || (aligned2(p) && chunk_tail_readable(p, rows, cols, ld));
+  };
+  const bool mid = algo == HCG_ALGO_AUTO && M > 16 && N > 32 && K <= (M > 32 ? 8192 : 4096);
+  const bool tiled_cols = mid && N <= 64 && 2 * M * K <= kCached && in_place(A, M, K, lda, K % 8 == 0);
   const bool use_narrow = algo == HCG_ALGO_NARROW ||
-                          (algo == HCG_ALGO_AUTO && rowstream_fits(A, lda, B, ldb, M, N, K));
-  // Otherwise M <= 16, and M <= 64 where the streaming kernel applies, is
-  // HBM-bound: B is streamed once through a skinny kernel instead of
-  // occupying only N/128 workgroups of the tiled kernel.  Rows 65..128 (the
-  // streaming kernel's eight row blocks) go to the tiled kernel, which splits
-  // K to fill the chip, when it reads B in place: fp16 us, streaming ->
-  // tiled: 128^3 5.9 -> 4.4, 128 x 512 x 512 9.2 -> 6.4, 128 x 2048 x 2048
-  // 14.1 -> 11.1, 128 x 8192 x 1024 16.2 -> 9.8, 128 x 16384 x 512 17.2 ->
-  // 7.3, 128 x 8192 x 8192 38.3 -> 35.7; with B's rows unaligned 128 x 3001
-  // x 1027 16.4 -> 14.0, 100 x 50257 x 1024 35.4 -> 23.6, 72 x 12289 x 4096
-  // 34.1 -> 27.8.  The streaming kernel led by at most 9% (80 x 4096 x 4096
-  // 16.6 against 18.0, 128 x 1001 x 2048 12.1 / 13.2).
-  const bool tiled_rows = M > 64 && ((aligned16(B) && ldb % 8 == 0) ||
-                                     (K > 0 && N > 0 && aligned2(B) && chunk_tail_readable(B, K, N, ldb)));
+                          (algo == HCG_ALGO_AUTO && !tiled_cols && rowstream_fits(A, lda, B, ldb, M, N, K));
+  const bool tiled_rows =
+      tiled_cols || ((M > 64 || (mid && N > 64 && 2 * N * K <= kCached)) && in_place(B, K, N, ldb, true));
   const bool use_skinny =
       !use_narrow && (algo == HCG_ALGO_SKINNY ||
                       (algo == HCG_ALGO_AUTO && (M <= 16 || (!tiled_rows && stream_fits(A, lda, B, ldb, M, N, K)))));

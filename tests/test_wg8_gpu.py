@@ -180,3 +180,15 @@ def test_summed_splits_match_the_reduce_launch(m, n, k):
             outs.append(c)
         torch.cuda.synchronize()
         assert torch.equal(outs[0], outs[1]), rnd
+
+
+# 17 to 64 rows and 33 to 64 columns: small operands take the tiled kernel,
+# larger ones and long K stream; both sides of each line.
+@pytest.mark.parametrize("m,n,k", [(16, 300, 500), (17, 65, 500), (32, 300, 4096), (32, 300, 4097),
+                                   (33, 300, 8192), (33, 300, 8193), (33, 1000, 999),
+                                   (64, 8192, 4096), (64, 8200, 4096), (64, 4001, 8191), (500, 32, 500),
+                                   (500, 33, 500), (17, 33, 100), (16, 33, 100), (4096, 64, 8192), (4104, 64, 8192),
+                                   (64, 64, 8200), (3001, 57, 777)])
+@pytest.mark.parametrize("pad", [0, 8])
+def test_few_rows_or_columns_either_route(m, n, k, pad):
+    _check(m, n, k, "float16", pad)
