@@ -2971,8 +2971,10 @@ int run_rowstream(const Scratch& sc, int dtype, const void* A, int64_t lda, cons
   a.a_bytes = a_dma ? (int)((((int64_t)M - 1) * lda + (int64_t)round_up(K, 8)) * 2) : 0;
   a.b_bytes = (int)((((int64_t)K - 1) * a.ldb + (int64_t)round_up(N, 8)) * 2);
   // One workgroup per CU (the ring takes a CU's LDS) walks the row blocks when
-  // there are over 1.25 per CU (see WALK).
-  const bool walk = a.splits == 1 && a_dma && (int64_t)4 * nrb >= (int64_t)5 * st->num_cus;
+  // there are over 1.25 per CU (see WALK); with 33 to 64 columns only up to
+  // K = 4096 (32768 x 40 x 4096 57.5 -> 55.9 us, 41267 x 40 x 6080 113.0 ->
+  // 114.1: a long block hides its ends).
+  const bool walk = a.splits == 1 && a_dma && (int64_t)4 * nrb >= (int64_t)5 * st->num_cus && (N <= 32 || K <= 4096);
   const dim3 grid((unsigned)(walk ? st->num_cus : nrb * a.splits));
   if (dtype == HCG_F16) {
     if (nb == 16) launch_rowstream<HCG_F16, 16>(a, !a_dma, short_ring, walk, grid, stream);
