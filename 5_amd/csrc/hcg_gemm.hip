@@ -10,7 +10,7 @@
 // matrix cores:
 //
 //   * gemm_dma_kernel -- compute-bound shapes.  TM x TN output tile per
-//     256-thread workgroup (256x256, 256x192, 128x256, 128x128 or 256x64, picked by
+//     256-thread workgroup (256x256, 256x192, 128x256 or 256x64, picked by
 //     size; 4 waves in 2x2, each (TM/2) x (TN/2) of MFMA 32x32x16 tiles),
 //     K step 32 through an LDS ring filled by direct global->LDS DMA loads
 //     (buffer_load ... lds; 256-row tiles move A two K steps at a time),

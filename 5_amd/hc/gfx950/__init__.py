@@ -200,14 +200,16 @@ def gemm(a: Any, b: Any, out: Any | None = None, *, algo: str = "auto", device: 
     computed, and copied back into ``out`` (created if None); the call then
     returns after the result is on the host.
 
-    ``algo``: "auto" (the library picks: the narrow streaming kernel for
-    N <= 64; the streaming kernel for M <= 64, and for M <= 128 when the
-    tiled kernel cannot read B in place; otherwise the LDS-tiled kernel
-    with a modelled tile shape and K split, with up to 128 rows or 64
-    columns past a multiple of 256 peeled off to a streaming kernel when
-    that saves a round of tiles.  Operands are read in place at any row
-    alignment; one whose last 16-byte piece cannot be read safely is
-    repacked, or goes through registers),
+    ``algo``: "auto" (the library picks: streaming kernels for N <= 64 and
+    for M <= 64, except that 33 columns or 17 rows and more of at most
+    64 MiB and a K of at most 8192 take the LDS-tiled kernel, and for
+    M <= 128 when the tiled kernel cannot read B in place; otherwise the
+    LDS-tiled kernel with a modelled tile shape and K split, with up to 128
+    rows or 64 columns past a multiple of 256 peeled off to a streaming
+    kernel when that saves a round of tiles.  Operands are read in place at
+    any row alignment; one whose last 16-byte piece cannot be read safely is
+    repacked, or goes through registers.  One transposed view, with M and N
+    above 64, is read in place too; other layouts are copied first),
     "tiled", "skinny", "narrow", "generic", or a fixed tile shape
     "tiled_256x256", "tiled_256x192", "tiled_128x256", "tiled_128x128",
     "tiled_256x64" (never split along K).
