@@ -55,6 +55,19 @@ __device__ __forceinline__ u32x4 load_row8_u16(const uint16_t* rowp, int64_t col
   return u32x4{w[0], w[1], w[2], w[3]};
 }
 
+// Origin plus offset in 64 bits: past 2^63 - 1 it wraps below zero, which is
+// outside every view.
+__device__ __forceinline__ int64_t tile_coord(int64_t origin, int64_t offset) {
+  return (int64_t)((uint64_t)origin + (uint64_t)offset);
+}
+
+// True iff row is inside [0, nrows) and all of columns col0 .. col0 + n - 1
+// inside [0, ncols).  The sum col0 + n is never formed: near 2^63 it would wrap
+// and pass.
+__device__ __forceinline__ bool chunk_inside(int64_t row, int64_t nrows, int64_t col0, int64_t ncols, int n) {
+  return row >= 0 && row < nrows && col0 >= 0 && col0 <= ncols - n;
+}
+
 // Bit e of the result is set iff column col0 + e (e < n) is inside
 // [0, ncols) and row is inside [0, nrows): the activity of a chunk of a
 // shape= load.
@@ -62,10 +75,8 @@ __device__ __forceinline__ uint32_t chunk_active_bits(int64_t row, int64_t nrows
                                                       int n) {
   if (row < 0 || row >= nrows) return 0u;
   uint32_t bits = 0;
-  for (int e = 0; e < n; ++e) {
-    const int64_t c = col0 + e;
-    if (c >= 0 && c < ncols) bits |= 1u << e;
-  }
+  for (int e = 0; e < n; ++e)
+    if (col0 >= -e && col0 < ncols - e) bits |= 1u << e;
   return bits;
 }
 

@@ -117,10 +117,10 @@ __global__ __launch_bounds__(256) void tile_load_kernel(TileJob j) {
     int64_t t, r, c0;
     decompose<T, I>(j, (I)at, t, r, c0);
     const int n = (int)min((int64_t)kN, j.tw - c0);
-    const int64_t row = j.origins[2 * t] + r;
-    const int64_t col = j.origins[2 * t + 1] + c0;
+    const int64_t row = hcg::tile_coord(j.origins[2 * t], r);
+    const int64_t col = hcg::tile_coord(j.origins[2 * t + 1], c0);
     const int64_t out_off = (t * j.th + r) * j.tw + c0;
-    const bool whole = n == kN && row >= 0 && row < j.rows && col >= 0 && col + kN <= j.cols;
+    const bool whole = n == kN && hcg::chunk_inside(row, j.rows, col, j.cols, kN);
     uint32_t active = whole ? kAll : hcg::chunk_active_bits(row, j.rows, col, j.cols, n);
     if (j.mask_in) active &= mask_bits<T>(j.mask_in + out_off, n);
     // Rows outside the view are never addressed (active is 0 for them).
@@ -168,10 +168,10 @@ __global__ __launch_bounds__(256) void tile_store_kernel(TileJob j) {
     int64_t t, r, c0;
     decompose<T, I>(j, (I)at, t, r, c0);
     const int n = (int)min((int64_t)kN, j.tw - c0);
-    const int64_t row = j.origins[2 * t] + r;
-    const int64_t col = j.origins[2 * t + 1] + c0;
+    const int64_t row = hcg::tile_coord(j.origins[2 * t], r);
+    const int64_t col = hcg::tile_coord(j.origins[2 * t + 1], c0);
     const int64_t in_off = (t * j.th + r) * j.tw + c0;
-    const bool whole = n == kN && row >= 0 && row < j.rows && col >= 0 && col + kN <= j.cols;
+    const bool whole = n == kN && hcg::chunk_inside(row, j.rows, col, j.cols, kN);
     uint32_t write = whole ? kAll : hcg::chunk_active_bits(row, j.rows, col, j.cols, n);
     if (write == 0) continue;
     const T* in = static_cast<const T*>(j.tiles_in) + in_off;

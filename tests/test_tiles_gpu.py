@@ -165,3 +165,26 @@ def test_more_chunks_than_one_pass_of_the_grid():
     covered = torch.zeros_like(src, dtype=torch.bool)
     covered[r[inside], c[inside]] = True
     assert torch.equal(dst, torch.where(covered, src, torch.zeros_like(src)))
+
+
+# Column origins a chunk (2, 4 or 8 elements) and less below 2^63, where the
+# end of the chunk is past it, and row and column origins at both ends of
+# int64: every element is outside the view.
+@pytest.mark.parametrize("name", ["float16", "float32", "int64"])
+def test_origins_at_the_ends_of_int64_are_outside_the_view(name):
+    import hc.gfx950 as g
+
+    top, bottom = (1 << 63) - 1, -(1 << 63)
+    origins = [[r, top - d] for r in (0, 3) for d in range(10)]
+    origins += [[1, bottom], [1, bottom + 7], [top, 0], [top - 1, 2], [bottom, 0], [top, top], [bottom, bottom]]
+    o = torch.tensor(origins, dtype=torch.int64, device=DEV)
+    n = len(origins)
+    guard = torch.full((8, 40), 5, dtype=DTYPES[name][0], device=DEV)
+    view = guard[2:6, 8:32]
+    print(f"case origins at the ends of int64 {name}", flush=True)
+    for shape in ((4, 16), (3, 21)):
+        for mask in (None, torch.ones((n, *shape), dtype=torch.bool, device=DEV)):
+            tiles, active = g.tile_load(view, o, shape, mask=mask, fill=-3)
+            assert not active.any() and (tiles == -3).all()
+            g.tile_store(view, o, torch.full_like(tiles, 9), mask=mask)
+            assert (guard == 5).all()
