@@ -164,17 +164,18 @@ class Const(Expr):
 class Symbol(Expr):
     """A named integer symbol (``sym.M``)."""
 
-    __slots__ = ("name", "_hash")
+    __slots__ = ("name",)
 
     def __init__(self, name: str) -> None:
         if not name or not name.isidentifier():
             raise ValueError(f"invalid symbol name {name!r}")
         self.name = name
-        self._hash = hash(("sym", name))
 
-    # (Symbols are the keys of every launch's bindings.)
+    # Symbols are the keys of every launch's bindings.  A string keeps its own
+    # hash; a copy of it in the symbol would travel with a pickle into
+    # processes whose strings hash differently.
     def __hash__(self) -> int:
-        return self._hash
+        return hash(self.name)
 
     def __eq__(self, other: object) -> bool:
         return True if self is other else Expr.__eq__(self, other)

@@ -6,6 +6,11 @@ equal.  CPU only."""
 
 from __future__ import annotations
 
+import os
+import pickle
+import subprocess
+import sys
+
 import pytest
 
 hypothesis = pytest.importorskip("hypothesis")
@@ -124,3 +129,30 @@ def test_binding_is_idempotent_and_conflicts_are_reported(m, other):
     if other != m:
         with pytest.raises(SymbolConflictError):
             b.bind(sym_of("M"), other)
+
+
+# Strings hash differently in every process: what a pickled symbol carries must
+# not depend on the process that wrote it.
+_OTHER_PROCESS = """
+import pickle, sys
+from hc.symbols import Bindings, SymbolConflictError, sym
+symbol, expr = pickle.load(sys.stdin.buffer)
+assert symbol == sym.M and hash(symbol) == hash(sym.M) and {sym.M: 1}[symbol] == 1
+bindings = Bindings()
+bindings.bind(sym.M, 40, source="a")
+assert expr.eval(bindings.freeze()) == 96
+try:
+    bindings.bind(symbol, 41, source="b")
+except SymbolConflictError:
+    pass
+else:
+    raise AssertionError("a conflicting extent was accepted")
+"""
+
+
+@pytest.mark.parametrize("seed", ["1", "2"])
+def test_pickled_symbols_work_in_another_process(seed):
+    data = pickle.dumps((sym_of("M"), ceil_div(sym_of("M"), 16) * 32))
+    env = {**os.environ, "PYTHONHASHSEED": seed, "PYTHONPATH": os.pathsep.join(p for p in sys.path if p)}
+    done = subprocess.run([sys.executable, "-c", _OTHER_PROCESS], input=data, env=env, capture_output=True, timeout=120)
+    assert done.returncode == 0, done.stderr.decode()
