@@ -84,6 +84,9 @@ class _PositionalBound(inspect.BoundArguments):
     def _signature(self) -> inspect.Signature:
         return inspect.Signature(list(inspect.signature(self._fn).parameters.values())[1:])
 
+    def __reduce__(self) -> Any:  # copies and pickles are plain BoundArguments
+        return inspect.BoundArguments, (self._signature, self.arguments)
+
 
 _VARIADIC = inspect.CO_VARARGS | inspect.CO_VARKEYWORDS
 

@@ -3,7 +3,9 @@ annotations follow the names they use."""
 
 from __future__ import annotations
 
+import copy
 import inspect
+import pickle
 
 import numpy as np
 import pytest
@@ -46,6 +48,16 @@ def test_binding_equals_inspect(fn, args, kwargs):
     got = _bind_arguments(fn, args, kwargs)
     assert got.arguments == want.arguments and list(got.arguments) == list(want.arguments)
     assert got.args == want.args and got.kwargs == want.kwargs and got.signature == want.signature
+
+
+@pytest.mark.parametrize("fn,args", [(_plain, (1, [2], 3)), (_defaults, (1,))])
+def test_bound_arguments_copy_and_pickle(fn, args):
+    """A lowering may keep a copy of the arguments it was given."""
+    bound = _bind_arguments(fn, args, {})
+    shallow = copy.copy(bound)
+    assert shallow == bound and shallow.arguments["a"] is bound.arguments["a"]
+    for other in (copy.deepcopy(bound), pickle.loads(pickle.dumps(bound))):
+        assert other == bound and other.args == args and other.signature == bound.signature
 
 
 @pytest.mark.parametrize("args,kwargs", [((1, 2), {}), ((1, 2, 3, 4), {}), ((1, 2, 3), {"c": 4}), ((1, 2, 3), {"d": 4})])
