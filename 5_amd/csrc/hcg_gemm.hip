@@ -3021,6 +3021,13 @@ int64_t fast_extent_b(int N, int K, int64_t ldb) {
   return ((int64_t)round_up(K, kTileK) * ldb + round_up(N, kTileN) + 8) * 2;
 }
 
+// True when both operands' byte offsets, tiles past their ends included, stay
+// below 2^31.
+bool fast_extents_fit(int M, int N, int K, int64_t lda, int64_t ldb) {
+  const int64_t kLimit = (int64_t)1 << 31;
+  return fast_extent_a(M, K, lda) < kLimit && fast_extent_b(N, K, ldb) < kLimit;
+}
+
 int run_tiled(const Scratch& sc, int dtype, const void* A, int64_t lda, const void* B, int64_t ldb,
               float* C, int64_t ldc, int M, int N, int K, bool force_generic, int force_shape) {
   DeviceState* st = sc.st;
@@ -3041,8 +3048,7 @@ int run_tiled(const Scratch& sc, int dtype, const void* A, int64_t lda, const vo
   const int64_t lda_p = a_ok ? lda : (int64_t)round_up(K, 8);
   const int64_t ldb_p = b_ok ? ldb : (int64_t)round_up(N, 8);
   const int64_t tiles = (int64_t)((M + kTileM - 1) / kTileM) * ((N + kTileN - 1) / kTileN);
-  const bool fits = fast_extent_a(M, K, lda_p) < kLimit && fast_extent_b(N, K, ldb_p) < kLimit &&
-                    tiles <= 0x7fffffff;
+  const bool fits = fast_extents_fit(M, N, K, lda_p, ldb_p) && tiles <= 0x7fffffff;
   // Aligned operands too large for 32-bit offsets from their base run the
   // WIDE form (per-tile / per-K-tile resources) when one 256-row panel of A
   // and one 32-row panel of B stay below 2^31 bytes.
@@ -3327,12 +3333,17 @@ int gemm_impl(int algo, int dtype, const void* A, int64_t lda, const void* B, in
   // 31.9 / 33.4.  With 17 to 32 columns they are even (4000 x 17 x 2000 8.6 /
   // 9.2), and 16 rows (16 x 4000 x 2000 8.2 / 8.9) or fewer stream.  Rows
   // 65 .. 128 go to the tiled kernel whatever B's size.  It needs the large
-  // operand readable in place.
+  // operand readable in place, and both within 32-bit offsets as they are
+  // strided: past those there are no small tiles and no K split, only
+  // gemm_dma_kernel's WIDE form or gemm_generic_kernel (32 x 4096 x 4096 out of
+  // rows of 300000 elements 15.7 us streaming, 42.9 WIDE; of 300001, 15.7 and
+  // 543 generic; 4096 x 64 x 4096 17.1 and 869).
   const int64_t kCached = (int64_t)64 << 20;
   const auto in_place = [](const void* p, int64_t rows, int64_t cols, int64_t ld, bool whole) {
     return (whole && aligned16(p) && ld % 8 == 0) || (aligned2(p) && chunk_tail_readable(p, rows, cols, ld));
   };
-  const bool mid = algo == HCG_ALGO_AUTO && M > 16 && N > 32 && K <= (M > 32 ? 8192 : 4096);
+  const bool mid = algo == HCG_ALGO_AUTO && M > 16 && N > 32 && K <= (M > 32 ? 8192 : 4096) &&
+                   fast_extents_fit((int)M, (int)N, (int)K, lda, ldb);
   const bool tiled_cols = mid && N <= 64 && 2 * M * K <= kCached && in_place(A, M, K, lda, K % 8 == 0);
   const bool use_narrow = algo == HCG_ALGO_NARROW ||
                           (algo == HCG_ALGO_AUTO && !tiled_cols && rowstream_fits(A, lda, B, ldb, M, N, K));

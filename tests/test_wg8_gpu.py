@@ -192,3 +192,26 @@ def test_summed_splits_match_the_reduce_launch(m, n, k):
 @pytest.mark.parametrize("pad", [0, 8])
 def test_few_rows_or_columns_either_route(m, n, k, pad):
     _check(m, n, k, "float16", pad)
+
+
+# Operands within the size rules above whose rows lie so far apart that they
+# span 2 GiB or more stream as before: the tiled kernel's small tiles and K
+# splits are for 32-bit offsets.  The same kernel gives the same bits.
+@pytest.mark.parametrize("m,n,k,lda,ldb,algo", [
+    (32, 512, 4096, 4096, 300000, "skinny"), (33, 520, 8000, 8000, 140001, "skinny"),
+    (64, 300, 4096, 4096, 262144, "skinny"), (4096, 64, 1000, 300000, 64, "narrow"),
+    (3000, 40, 513, 400001, 40, "narrow")])
+def test_few_rows_or_columns_of_a_wide_matrix_stream(m, n, k, lda, ldb, algo):
+    import hc.gfx950 as g
+
+    print(f"case wide rows m={m} n={n} k={k} lda={lda} ldb={ldb}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(m + n + k)
+    a = torch.full((m, lda), float("nan"), dtype=torch.float16, device=DEV)[:, :k]
+    b = torch.full((k, ldb), float("nan"), dtype=torch.float16, device=DEV)[:, :n]
+    a.copy_(torch.randn(a.shape, generator=gen, device=DEV))
+    b.copy_(torch.randn(b.shape, generator=gen, device=DEV))
+    got = g.gemm(a, b)
+    assert torch.equal(got, g.gemm(a, b, algo=algo))
+    want = a.double() @ b.double()
+    # 32-bit sums of k exact products, in any order: each within k units of 2^-24 of the sum of magnitudes.
+    assert ((got - want).abs() <= k * 2.0**-24 * (a.double().abs() @ b.double().abs())).all()
