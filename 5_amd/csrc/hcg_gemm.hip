@@ -2432,7 +2432,8 @@ int launch_generic(const TiledArgs& a, bool vec_a, bool vec_b, hipStream_t strea
 // wg8): 256^3 5.2 -> 3.7 (64x64), 1000^3 14.4 -> 7.8 (64x64),
 // 8192 x 128 x 2048 21.0 -> 8.8 (64x64), 512 x 4096 x 4096 37.9 -> 22.4
 // (64x128), 2048^3 23.2 -> 18.2 (128x128), 2500^3 38.7 -> 35.7 (128x256);
-// 128 x 128 tiles of gemm_dma_kernel were never the fastest and are gone,
+// 128 x 128 tiles of gemm_dma_kernel were never the fastest (only its WIDE
+// form, which splits no K, keeps them),
 // its 256-row tiles stay ahead from about 256 of them (3000^3 54.4 against
 // 78.2) and its 128x256 tiles, two workgroups per CU, where a CU takes two
 // or more (8192 x 8192 x 256 60.5 against 70.5).
@@ -2455,10 +2456,14 @@ constexpr TileShape kTileShapes[] = {
     // Transposed operands only (gemm_dma_kernel's four waves are ahead on
     // row-major ones: 4096^3 bf16 98.5 us against 103.4).
     {256, 256, 1, 32, true, 8.04f, 0.460f, 0.70f},
+    // gemm_dma_kernel's WIDE form only, which no wg8 shape has (4096 x 128 x 512
+    // 6.8 us, on 128x256 tiles 10.0; 100 x 4096 x 4096 38.3 / 43.7).
+    {128, 128, 2, 32, false, 2.2f, 0.275f, 0.30f},
 };
 constexpr int kNumTileShapes = sizeof(kTileShapes) / sizeof(kTileShapes[0]);
 constexpr int kNarrowShape = 4;
 constexpr int kTransShape = 8;
+constexpr int kWideShape = 9;
 constexpr double kLaunchUs = 2.0;
 
 // Picks the tile shape and K split with the least modelled time.
@@ -2543,7 +2548,9 @@ TilePlan plan_tiles(int num_cus, int M, int N, int K, int force_shape, bool allo
   for (int i = 0; i < kNumTileShapes; ++i) {
     const TileShape& t = kTileShapes[i];
     if (force_shape >= 0 ? i != force_shape : i == kNarrowShape && N > 64) continue;
-    if (force_shape < 0 && (ops == kWide ? t.wg8 : ops == kTrans ? !t.wg8 : i == kTransShape)) continue;
+    if (force_shape < 0 &&
+        (ops == kWide ? t.wg8 : ops == kTrans ? !t.wg8 : i == kTransShape || i == kWideShape))
+      continue;
     if (plan_tile_count(t, M, N) * 64 > 0x7fffffff) continue;
     for (int c = 0; c < (forced_splits > 0 ? 1 : (int)(sizeof(kSplitCandidates) / sizeof(int))); ++c) {
       const int splits = forced_splits > 0 ? forced_splits : kSplitCandidates[c];
@@ -2625,7 +2632,8 @@ int launch_dma(const FastArgs& a, int shape, hipStream_t stream) {
   switch (shape) {
     case 0: gemm_dma_kernel<DT, 256, 256, 4, WIDE, KT, kA2><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
     case 1: gemm_dma_kernel<DT, 256, 192, 4, WIDE, KT, kA2><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;
-    case 3:  // (WIDE only: 128x128 tiles otherwise run on wg8)
+    case 3:  // (WIDE only, forced or planned: 128x128 tiles otherwise run on wg8)
+    case kWideShape:
       if constexpr (WIDE) gemm_dma_kernel<DT, 128, 128, 3, WIDE, KT><<<grid, block, 0, stream>>>(HCG_STAMPED(a));
       break;
     case 4: gemm_dma_kernel<DT, 256, 64, 4, WIDE, KT, kA2><<<grid, block, 0, stream>>>(HCG_STAMPED(a)); break;

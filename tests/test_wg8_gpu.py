@@ -215,3 +215,36 @@ def test_few_rows_or_columns_of_a_wide_matrix_stream(m, n, k, lda, ldb, algo):
     want = a.double() @ b.double()
     # 32-bit sums of k exact products, in any order: each within k units of 2^-24 of the sum of magnitudes.
     assert ((got - want).abs() <= k * 2.0**-24 * (a.double().abs() @ b.double().abs())).all()
+
+
+def _kernels_of(fn):
+    """Names of the kernels a call runs."""
+    from torch.profiler import ProfilerActivity, profile
+
+    fn()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as prof:
+        fn()
+        torch.cuda.synchronize()
+    return [e.name for e in prof.events() if e.device_type == torch.autograd.DeviceType.CUDA]
+
+
+# Rows so far apart that an operand spans 2 GiB: the WIDE form of
+# gemm_dma_kernel, whose 128x128 tiles are the fastest while the larger ones
+# leave CUs idle.
+@pytest.mark.parametrize("m,n,k,lda,tile", [(4097, 128, 512, 300000, "128, 128"), (4096, 1000, 40, 300000, "128, 128"),
+                                            (16000, 1000, 64, 80000, "128, 256"),
+                                            (4096, 4096, 1024, 300000, "256, 256")])
+def test_wide_tiles_by_size(m, n, k, lda, tile):
+    import hc.gfx950 as g
+
+    print(f"case wide tiles m={m} n={n} k={k} lda={lda}", flush=True)
+    rng = np.random.default_rng(m + n + k)
+    ai, bi = rng.integers(-4, 5, size=(m, k)), rng.integers(-4, 5, size=(k, n))
+    a = torch.full((m, lda), float("nan"), dtype=torch.float16, device=DEV)[:, :k]
+    a.copy_(torch.from_numpy(ai.astype(np.float32)))
+    b = torch.from_numpy(bi.astype(np.float32)).to(DEV).half()
+    out = torch.empty(m, n, device=DEV)
+    names = _kernels_of(lambda: g.gemm(a, b, out=out))
+    assert np.array_equal(out.cpu().numpy(), (ai.astype(np.float64) @ bi.astype(np.float64)).astype(np.float32))
+    assert any(f"gemm_dma_kernel<0, {tile}, " in name for name in names), names
