@@ -2233,17 +2233,12 @@ int current_device_state(DeviceState** out) {
 // The caller holds st->ws_mutex from this call until every kernel that uses
 // *out is enqueued: another thread's call (on the same stream, needing more
 // bytes, or evicting the slot) frees the buffer, and hipFree waits only for
-// work already enqueued.  With `counters`, also returns the buffer's arrival
-// counters, first clearing them (a fill kernel on `stream`, never a memset,
-// so a capture records a kernel node) when the buffer is new or the stream
-// is being captured (a graph must not depend on what ran before a replay).
-int stream_workspace(DeviceState* st, hipStream_t stream, size_t bytes, void** out,
+// work already enqueued.  `capturing`: the stream is being captured.  With
+// `counters` (eager calls only: a graph must not depend on what ran before a
+// replay), also returns the buffer's arrival counters, first clearing them
+// when the buffer is new.
+int stream_workspace(DeviceState* st, hipStream_t stream, bool capturing, size_t bytes, void** out,
                      unsigned** counters = nullptr) {
-  // The null stream is never captured (and querying it during another
-  // stream's capture is itself an error), so only real streams are asked.
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  if (stream != nullptr) HCG_HIP_CHECK(hipStreamIsCapturing(stream, &capture));
-  const bool capturing = capture == hipStreamCaptureStatusActive;
   Workspace* w = nullptr;
   for (auto& cand : st->ws)
     if (cand.ptr && cand.stream == (void*)stream) w = &cand;
@@ -2281,7 +2276,7 @@ int stream_workspace(DeviceState* st, hipStream_t stream, size_t bytes, void** o
   *out = static_cast<char*>(w->ptr) + kStCounterBytes;
   if (counters) {
     *counters = static_cast<unsigned*>(w->ptr);
-    if (!w->counters_zeroed || capturing) {
+    if (!w->counters_zeroed) {
       constexpr int n = kStCounterBytes / 4;
       fill_zero_kernel<<<(n + 255) / 256, 256, 0, stream>>>(static_cast<float*>(w->ptr), n, 1, n);
       HCG_HIP_CHECK(hipGetLastError());
@@ -2342,6 +2337,30 @@ struct Scratch {
   void* fixed = nullptr;
   size_t cap = 0;
 
+  // Whether the stream is being captured, asked once per call.  (The null
+  // stream never is, and querying it during another stream's capture is itself
+  // an error, so only real streams are asked.)
+  bool capturing() const {
+    if (!asked) {
+      hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+      if (stream != nullptr) error = hipStreamIsCapturing(stream, &status);
+      captured = status == hipStreamCaptureStatusActive;
+      asked = true;
+    }
+    return captured;
+  }
+  // Whether a block's last workgroup may sum its K splits (hcg_splitsum.h): that
+  // takes arrival counters at zero.  The fixed buffer has none, and in a graph
+  // they would have to be cleared before every such launch, by a kernel that
+  // costs more than the second launch that sums the partials instead, in the
+  // same order (replays, fp16 us, fill + fused / reduce launch: 512 x 512 x 16384
+  // 19.8 / 16.9, 128 x 128 x 1024 7.3 / 6.4, 300 x 5 x 900 7.9 / 6.8,
+  // 16 x 4096 x 4096 11.9 / 10.3; 128 x 8192 x 8192 37.5 / 36.8).
+  bool counters() const { return !fixed && !capturing(); }
+
+  mutable bool asked = false, captured = false;
+  mutable hipError_t error = hipSuccess;
+
   // Bytes available for split partials once `used` bytes are taken.
   size_t room(size_t used) const {
     if (!fixed) return SIZE_MAX;
@@ -2349,10 +2368,9 @@ struct Scratch {
   }
 };
 
-// `counters` (optional) receives the workspace's arrival counters, or null
-// for the fixed buffer, which has none.
+// `counters` (optional; only where sc.counters()) receives the workspace's
+// arrival counters.
 int get_scratch(const Scratch& sc, size_t bytes, void** out, unsigned** counters = nullptr) {
-  if (counters) *counters = nullptr;
   if (sc.fixed) {
     if (bytes > sc.cap)
       return set_error(HCG_EINVAL,
@@ -2362,7 +2380,9 @@ int get_scratch(const Scratch& sc, size_t bytes, void** out, unsigned** counters
     *out = sc.fixed;
     return HCG_OK;
   }
-  return stream_workspace(sc.st, sc.stream, bytes, out, counters);
+  const bool capturing = sc.capturing();
+  HCG_HIP_CHECK(sc.error);
+  return stream_workspace(sc.st, sc.stream, capturing, bytes, out, counters);
 }
 
 // Largest split count (at most `splits`, at least 1) whose partials of
@@ -2806,9 +2826,10 @@ int run_skinny(const Scratch& sc, int dtype, const void* A, int64_t lda, const v
     // Whole column blocks when the last workgroup sums them; else rows of N.
     const int nblocks = (N + kStN - 1) / kStN;
     const size_t fused_sz = (size_t)a.splits * 16 * a.rblocks * nblocks * kStN * sizeof(float);
-    const bool fuse = !sc.fixed && a.splits > 1 && stream_can_fuse(a.rblocks) && a.splits <= hcg::kMaxSummedSplits &&
+    const bool fuse = a.splits > 1 && stream_can_fuse(a.rblocks) && a.splits <= hcg::kMaxSummedSplits &&
                       a.splits * 16 * a.rblocks * kStN * 4 <= hcg::kMaxSummedBytes &&
-                      nblocks * hcg::kSplitCounterStride * 4 <= kStCounterBytes && fused_sz < ((size_t)1 << 31);
+                      nblocks * hcg::kSplitCounterStride * 4 <= kStCounterBytes && fused_sz < ((size_t)1 << 31) &&
+                      sc.counters();
     const size_t p_sz = fuse           ? fused_sz
                         : a.splits > 1 ? (size_t)a.splits * 16 * a.rblocks * (size_t)N * sizeof(float)
                                        : 0;
@@ -2817,7 +2838,7 @@ int run_skinny(const Scratch& sc, int dtype, const void* A, int64_t lda, const v
       unsigned* counters = nullptr;
       const int rc = get_scratch(sc, a_sz + p_sz, &ws, fuse ? &counters : nullptr);
       if (rc != HCG_OK) return rc;
-      if (fuse && counters) {
+      if (fuse) {
         a.counters = counters;
         a.ws_bytes = (int)p_sz;
       }
@@ -2954,9 +2975,10 @@ int run_rowstream(const Scratch& sc, int dtype, const void* A, int64_t lda, cons
   // With small partials the last workgroup of a row block sums them.
   const int nb = N <= 16 ? 16 : N <= 32 ? 32 : 64;
   const size_t fused_sz = (size_t)a.splits * nrb * kRsRows * nb * sizeof(float);
-  const bool fuse = !sc.fixed && a.splits > 1 && a.splits <= hcg::kMaxSummedSplits &&
+  const bool fuse = a.splits > 1 && a.splits <= hcg::kMaxSummedSplits &&
                     a.splits * kRsRows * nb * 4 <= hcg::kMaxSummedBytes &&
-                    nrb * hcg::kSplitCounterStride * 4 <= kStCounterBytes && fused_sz < ((size_t)1 << 31);
+                    nrb * hcg::kSplitCounterStride * 4 <= kStCounterBytes && fused_sz < ((size_t)1 << 31) &&
+                    sc.counters();
   const size_t p_sz = fuse ? fused_sz : a.splits > 1 ? (size_t)a.splits * M * N * sizeof(float) : 0;
   if (b_sz + p_sz > 0) {
     void* ws = nullptr;
@@ -3090,9 +3112,9 @@ int run_tiled(const Scratch& sc, int dtype, const void* A, int64_t lda, const vo
   // Explicit tile shapes run without a K split; "auto" and "tiled" may split.
   const size_t room = sc.room(a_sz + b_sz);
   TilePlan plan = plan_tiles(st->num_cus, M, N, K, force_shape, force_shape < 0, nullptr, room);
-  if (plan.fused && sc.fixed) {
-    // The fixed buffer has no counters: the same splits by a second launch
-    // (the same sums in the same order) where their partials fit.
+  if (plan.fused && !sc.counters()) {
+    // The same splits by a second launch (the same sums in the same order)
+    // where their partials fit.
     if ((size_t)plan.splits * M * N * sizeof(float) <= room)
       plan.fused = false;
     else
@@ -3188,7 +3210,8 @@ int run_trans(const Scratch& sc, int dtype, bool a_t, const void* A, int64_t lda
            (aligned2(p) && chunk_tail_readable(p, rows, cols, ld));
   };
   if (!readable(A, ar, ac, lda, !a_t) || !readable(B, br, bc, ldb, b_t)) return HCG_EDECLINED;
-  const TilePlan plan = plan_tiles(sc.st->num_cus, (int)M, (int)N, (int)K, -1, true, nullptr, sc.room(0), kTrans);
+  TilePlan plan = plan_tiles(sc.st->num_cus, (int)M, (int)N, (int)K, -1, true, nullptr, sc.room(0), kTrans);
+  plan.fused = plan.fused && sc.counters();  // else the same splits by a second launch
   const TileShape& ts = kTileShapes[plan.shape];
   hcg::wg8::Args a{};
   a.A = static_cast<const uint16_t*>(A);
@@ -3285,8 +3308,8 @@ Peel plan_peel(const DeviceState* st, const void* A, int64_t lda, const void* B,
   return p;
 }
 
-// `fixed` / `fixed_bytes`: a caller-owned scratch buffer that replaces the
-// stream's library workspace (nothing is allocated); null for the default.
+// no_alloc: scratch from the device's fixed array, which replaces the stream's
+// library workspace (nothing is allocated).
 int gemm_impl(int algo, int dtype, const void* A, int64_t lda, const void* B, int64_t ldb,
               float* C, int64_t ldc, int64_t M, int64_t N, int64_t K, void* stream_ptr,
               bool no_alloc = false) {

@@ -248,3 +248,41 @@ def test_wide_tiles_by_size(m, n, k, lda, tile):
     names = _kernels_of(lambda: g.gemm(a, b, out=out))
     assert np.array_equal(out.cpu().numpy(), (ai.astype(np.float64) @ bi.astype(np.float64)).astype(np.float32))
     assert any(f"gemm_dma_kernel<0, {tile}, " in name for name in names), names
+
+
+# K splits whose partials an eager call sums in its last workgroups (tiled,
+# transposed, streaming, narrow): captured, a second launch sums them, in the
+# same order and with nothing to clear.
+@pytest.mark.parametrize("m,n,k,which", [(512, 512, 16384, ""), (103, 254, 779, ""), (300, 200, 8192, "a"),
+                                         (300, 200, 8192, "b"), (16, 4096, 4096, ""), (31, 4099, 5000, ""),
+                                         (2048, 24, 12000, ""), (300, 5, 900, "")])
+def test_captured_splits_match_eager_and_clear_nothing(m, n, k, which):
+    import hc.gfx950 as g
+
+    print(f"case captured splits m={m} n={n} k={k} {which}", flush=True)
+    x = torch.empty((k, m) if which == "a" else (m, k), dtype=torch.float16, device=DEV)
+    y = torch.empty((n, k) if which == "b" else (k, n), dtype=torch.float16, device=DEV)
+    a, b = x.t() if which == "a" else x, y.t() if which == "b" else y
+    out, eager = torch.empty(m, n, device=DEV), torch.empty(m, n, device=DEV)
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        g.gemm(a, b, out=eager)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        for _ in range(2):  # back to back: the second's partials overwrite the first's
+            g.gemm(a, b, out=out)
+    names = _kernels_of(graph.replay)
+    assert any("gemm" in name for name in names) and not any("fill_zero" in name for name in names), names
+    for seed in range(4):
+        gen = torch.Generator(device=DEV).manual_seed(seed)
+        x.copy_(torch.randn(x.shape, generator=gen, device=DEV))
+        y.copy_(torch.randn(y.shape, generator=gen, device=DEV))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            g.gemm(a, b, out=eager)
+        torch.cuda.synchronize()
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), seed
