@@ -3188,11 +3188,25 @@ int run_tiled(const Scratch& sc, int dtype, const void* A, int64_t lda, const vo
   return launch_reduce(f.ws, C, ldc, M, N, M, f.splits, aligned16(C) && ldc % 4 == 0, stream);
 }
 
+// Whether B stored transposed is better copied to row-major first.  In place
+// every tile reads it in 64-byte pieces of rows 2 K bytes apart, which costs the
+// K loop 3% and, with K, up to a quarter (8192^3 fp16 912 us; A stored
+// transposed 824); a copy costs the same whatever M, so many rows pay for it.
+// us, copied / in place, (M, N, K): (16384, 4096, 4096) 498 / 467, (32768, 4096,
+// 4096) 924 / 938, (65536, 4096, 4096) 1777 / 1930, (65536, 4096, 1024) 556 / 557,
+// (131072, 2048, 2048) 997 / 1080, (16384, 8192, 8192) 1902 / 1811, (32768, 8192,
+// 8192) 3535 / 3644, (8192, 4096, 16384) 1097 / 1017, (16384, 4096, 16384) 1894 /
+// 2017, (32768, 4096, 16384) 3526 / 4114; the line is a fit to 65 such points,
+// within 1.5% of the faster one on 64 of them and 4% on the other.  From K = 16384 on the copy slows too
+// (8192 x 8192 x 32768 4505 / 4116).  A stored transposed lost nowhere.
+bool trans_b_copied(int64_t M, int64_t K) { return (double)M * ((K < 16384 ? K : 16384) + 2250) >= 2.1e8; }
+
 // The tiled kernel on a transposed operand, read where it lies: A stored as
 // K x M (a_t) or B stored as N x K (b_t), not both.  HCG_EDECLINED, with
 // nothing launched, for what only the row-major kernels take: few rows or
 // columns (streaming kernels), operands whose last 16-byte piece cannot be
-// read safely, offsets past 2^31.
+// read safely, offsets past 2^31, and B transposed under many rows
+// (trans_b_copied).
 int run_trans(const Scratch& sc, int dtype, bool a_t, const void* A, int64_t lda, bool b_t, const void* B,
               int64_t ldb, float* C, int64_t ldc, int64_t M, int64_t N, int64_t K) {
   const int64_t kLimit = (int64_t)1 << 31;
@@ -3201,7 +3215,7 @@ int run_trans(const Scratch& sc, int dtype, bool a_t, const void* A, int64_t lda
   };
   // Stored rows and columns.
   const int64_t ar = a_t ? K : M, ac = a_t ? M : K, br = b_t ? N : K, bc = b_t ? K : N;
-  if (a_t == b_t || M <= 64 || N <= 64 || lda >= kLimit || ldb >= kLimit || extent(ar, ac, lda) >= kLimit ||
+  if (a_t == b_t || M <= 64 || N <= 64 || (b_t && trans_b_copied(M, K)) || lda >= kLimit || ldb >= kLimit || extent(ar, ac, lda) >= kLimit ||
       extent(br, bc, ldb) >= kLimit)
     return HCG_EDECLINED;
   const bool k8 = K % 8 == 0;

@@ -110,7 +110,8 @@ int hcg_gemm_noalloc(int dtype, const void* A, int64_t lda, const void* B, int64
  * transposing copy.  HCG_EDECLINED, with nothing launched and no error text,
  * when the call needs a row-major copy instead: both or neither operand
  * transposed, M <= 64 or N <= 64 (the streaming kernels'), K == 0, an operand
- * whose last 16-byte piece cannot be read safely, or offsets past 2^31.  No
+ * whose last 16-byte piece cannot be read safely, offsets past 2^31, or B
+ * transposed under so many rows (32000 at K = 4096) that a copy pays.  No
  * counterpart in the reference, whose buffers are row-major. */
 int hcg_gemm_trans(int dtype, int a_trans, const void* A, int64_t lda, int b_trans, const void* B, int64_t ldb,
                    float* C, int64_t ldc, int64_t M, int64_t N, int64_t K, void* stream);

@@ -286,3 +286,31 @@ def test_captured_splits_match_eager_and_clear_nothing(m, n, k, which):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager), seed
+
+
+# Under many rows a transposed B is copied to row-major first (both sides of the
+# line at three K; A stored transposed never is).
+@pytest.mark.parametrize("m,n,k,copied", [(64000, 66, 1024, False), (64300, 66, 1024, True), (32900, 65, 4096, False),
+                                          (33200, 65, 4096, True), (11200, 100, 16400, False),
+                                          (11300, 100, 16400, True)])
+def test_transposed_b_under_many_rows_is_copied(m, n, k, copied):
+    import hc.gfx950 as g
+    from hc.gfx950 import _native
+
+    print(f"case transposed b under many rows m={m} n={n} k={k}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(m + k)
+    a = torch.randint(-3, 4, (m, k), generator=gen, device=DEV).half()
+    bt = torch.randint(-3, 4, (n, k), generator=gen, device=DEV).half()
+    c = torch.full((m, n), float("nan"), device=DEV)
+    lib = _native.load()
+    rc = lib.hcg_gemm_trans(_native.HCG_F16, 0, a.data_ptr(), k, 1, bt.data_ptr(), k, c.data_ptr(), n, m, n, k,
+                            torch.cuda.current_stream().cuda_stream or None)
+    assert rc == (_native.HCG_EDECLINED if copied else _native.HCG_OK), _native.last_error(lib)
+    got = g.gemm(a, bt.t())
+    want = torch.empty_like(c)  # |sums| < 2^24: exact in float32 in any order
+    for i in range(0, m, 8192):
+        want[i : i + 8192] = a[i : i + 8192].float() @ bt.t().float().contiguous()
+    assert torch.equal(got, want)
+    assert torch.isnan(c).all() if copied else torch.equal(c, want)
+    at = a[:8200].t().contiguous().t()
+    assert torch.equal(g.gemm(at, bt.t().contiguous()), want[:8200])
