@@ -1218,8 +1218,8 @@ __global__ __launch_bounds__(kSkinnyThreads) void gemm_skinny_kernel(SkinnyArgs 
 // feeds R MFMAs.  Each block's 16x32 slice of a stage arrives by one more
 // DMA instruction (block rb from wave rb % 4).
 //
-// Split-K partials go to a workspace.  Where they are small (R <= 4,
-// kMaxSummedBytes) the last workgroup of a column block to arrive sums them in
+// Split-K partials go to a workspace.  Where they are few and small
+// (stream_summed_splits) the last workgroup of a column block to arrive sums them in
 // order s = 0..S-1 and writes C (sum_splits, hcg_splitsum.h).  Otherwise (and
 // for the allocation-free entry point, which has no counters) they are rows
 // [splits][16 R][N] that stream_reduce_kernel sums in a second launch, in the
@@ -1232,9 +1232,14 @@ constexpr int kStBBytes = kStStep * kStN * 2;  // 8 KB
 constexpr int kStABytes = 16 * kStStep * 2;    // 1 KB per 16-row block of A
 constexpr int kStMaxRowBlocks = 8;              // M <= 128
 constexpr int kStMaxSplits = 16;      // partials stream_reduce_kernel holds in registers
-// Row blocks up to which the last workgroup of a column block sums its K
-// splits (hcg_splitsum.h); R = 8's partials are 64 KB each.
-constexpr bool stream_can_fuse(int R) { return R <= 4; }
+// K splits up to which the last workgroup of a column block sums them
+// (hcg_splitsum.h): partials are 8 KB for one row block, loaded eight at a time;
+// 16 KB for two, 32 KB for four.  fp16 us, second launch / summed in the kernel:
+// one row block 16 x 1000 x 2050 (8 splits) 6.7 / 6.3, 16 x 1000 x 2560 (10)
+// 6.6 / 6.8, 8 x 2048 x 2560 (10) 6.7 / 7.4, 16 x 1000 x 4096 (16) 7.0 / 7.9; two
+// 32 x 6000 x 6000 (5) 19.3 / 19.0, 31 x 4099 x 5000 (7) 17.6 / 18.0; four
+// 48 x 8200 x 8192 (3) 36.1 / 36.0, 64 x 8192 x 8192 (4) 30.0 / 30.3.
+constexpr int stream_summed_splits(int R) { return R == 1 ? 8 : R == 2 ? 6 : R == 4 ? 3 : 0; }
 constexpr int kStCounterBytes = 16384;  // arrival counters ahead of each workspace: 256 of them, 64 bytes apart
 constexpr int kStMaxSplitsLoop = 256;  // K splits at all (more than 16: split_reduce_kernel)
 
@@ -1588,7 +1593,7 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(StreamArgs g) {
   // column l%16 of the block.
   const int ocol = n0 + wave * kColsPerWave + (lane & 15);
   bool to_c = g.splits == 1;
-  if constexpr (stream_can_fuse(R)) {
+  if constexpr (stream_summed_splits(R) > 0) {
     if (!to_c && g.counters != nullptr) {
       to_c = hcg::sum_splits<R * kBlocks, 256>(reinterpret_cast<f32x4(&)[R * kBlocks]>(acc),
                                                make_rsrc(g.ws, g.ws_bytes), (g.N + NB - 1) / NB, nb, g.splits, split,
@@ -2826,8 +2831,7 @@ int run_skinny(const Scratch& sc, int dtype, const void* A, int64_t lda, const v
     // Whole column blocks when the last workgroup sums them; else rows of N.
     const int nblocks = (N + kStN - 1) / kStN;
     const size_t fused_sz = (size_t)a.splits * 16 * a.rblocks * nblocks * kStN * sizeof(float);
-    const bool fuse = a.splits > 1 && stream_can_fuse(a.rblocks) && a.splits <= hcg::kMaxSummedSplits &&
-                      a.splits * 16 * a.rblocks * kStN * 4 <= hcg::kMaxSummedBytes &&
+    const bool fuse = a.splits > 1 && a.splits <= stream_summed_splits(a.rblocks) &&
                       nblocks * hcg::kSplitCounterStride * 4 <= kStCounterBytes && fused_sz < ((size_t)1 << 31) &&
                       sc.counters();
     const size_t p_sz = fuse           ? fused_sz
@@ -2914,6 +2918,13 @@ bool rowstream_fits(const void* A, int64_t lda, const void* B, int64_t ldb, int6
          ((int64_t)round_up(K, kRsStep) * ldb_use + 64) * 2 < ((int64_t)1 << 31);
 }
 
+// K splits up to which the last workgroup of a row block sums them: partials are
+// 4 KB (16 columns), 8 KB (32) or 16 KB (64).  fp16 us, second launch / summed in
+// the kernel: 200 x 12 x 8192 (16 splits) 7.1 / 6.5; 400 x 24 x 4096 (8) 7.3 / 6.7,
+// 400 x 24 x 5120 (10) 7.4 / 7.4, 400 x 24 x 8192 (16) 7.7 / 8.2; 2048 x 57 x 12001
+// (8) 19.0 / 17.5.
+constexpr int rowstream_summed_splits(int nb) { return nb == 16 ? hcg::kMaxSummedSplits : 8; }
+
 template <int DT, int NB>
 void launch_rowstream(const RowStreamArgs& a, bool ua, bool short_ring, bool walk, dim3 grid, hipStream_t stream) {
   if constexpr (NB <= 32) {
@@ -2975,8 +2986,7 @@ int run_rowstream(const Scratch& sc, int dtype, const void* A, int64_t lda, cons
   // With small partials the last workgroup of a row block sums them.
   const int nb = N <= 16 ? 16 : N <= 32 ? 32 : 64;
   const size_t fused_sz = (size_t)a.splits * nrb * kRsRows * nb * sizeof(float);
-  const bool fuse = a.splits > 1 && a.splits <= hcg::kMaxSummedSplits &&
-                    a.splits * kRsRows * nb * 4 <= hcg::kMaxSummedBytes &&
+  const bool fuse = a.splits > 1 && a.splits <= rowstream_summed_splits(nb) &&
                     nrb * hcg::kSplitCounterStride * 4 <= kStCounterBytes && fused_sz < ((size_t)1 << 31) &&
                     sc.counters();
   const size_t p_sz = fuse ? fused_sz : a.splits > 1 ? (size_t)a.splits * M * N * sizeof(float) : 0;

@@ -23,12 +23,6 @@ typedef float split_f32x4 __attribute__((ext_vector_type(4)));
 // 16384 in 32 tiles and 8 splits: 19.4 -> 18.6 us).
 constexpr int kSplitCounterStride = 16;
 constexpr int kMaxSummedSplits = 16;
-// Where no model decides: bytes of a block's partials (all splits) up to which
-// its last workgroup is faster than a second launch.  16 x 8191 x 8192 (32 KB)
-// 31.9 -> 30.6 us, 64 x 8192 x 8192 (128 KB) 30.3 -> 30.1, 48 x 4096 x 4096
-// (256 KB) 12.1 -> 14.9; 4096 x 64 x 1024 (64 KB) 9.1 -> 7.4, 4096 x 13 x 8192
-// (16 KB) 15.4 -> 14.3.
-constexpr int kMaxSummedBytes = 128 << 10;
 
 // v: this thread's P pieces of split `split`'s partial of block `block` (of
 // `blocks`).  The workspace holds [splits][blocks][P][THREADS] pieces: writer

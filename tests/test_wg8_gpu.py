@@ -154,15 +154,33 @@ def test_narrow_kernel_walks_row_blocks(m, n, k, dtype):
     _check(m, n, k, dtype, 3 if dtype == "float16" else 8)
 
 
+def _kernels_of(fn):
+    """Names of the kernels a call runs."""
+    from torch.profiler import ProfilerActivity, profile
+
+    fn()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as prof:
+        fn()
+        torch.cuda.synchronize()
+    return [e.name for e in prof.events() if e.device_type == torch.autograd.DeviceType.CUDA]
+
+
 # K splits summed by a block's last workgroup against the same partials summed
 # by a second launch, which hcg_gemm_noalloc keeps: in the same order, so bit
 # for bit, with new operands every round (a stale partial would show).  The
-# streaming kernel with N not a multiple of 4, of 128 and with four row blocks;
-# the narrow kernel with 16, 32 and 64 columns.
-@pytest.mark.parametrize("m,n,k", [(16, 8191, 8192), (1, 1001, 4096), (31, 4099, 2048), (64, 8192, 8192),
-                                   (40, 3001, 8191), (4096, 13, 8192), (2048, 24, 12000), (4096, 64, 1024),
-                                   (300, 5, 900), (1000, 33, 4001)])
-def test_summed_splits_match_the_reduce_launch(m, n, k):
+# streaming kernel with one, two and four row blocks at their most splits, N
+# ragged or not; the narrow kernel with 16, 32 and 64 columns; and one split
+# more than each takes, where both calls run the second launch.
+@pytest.mark.parametrize("m,n,k,kernel,summed", [
+    (16, 8191, 8192, "stream", True), (1, 1001, 2050, "stream", True), (16, 1000, 2560, "stream", False),
+    (31, 5001, 5000, "stream", True), (31, 4099, 5000, "stream", False),
+    (40, 9001, 8191, "stream", True), (64, 8192, 8200, "stream", False),
+    (4096, 13, 8192, "rowstream", True), (200, 12, 8192, "rowstream", True), (300, 5, 900, "rowstream", True),
+    (2048, 24, 12000, "rowstream", True), (400, 24, 5120, "rowstream", False),
+    (2048, 57, 12001, "rowstream", True), (1000, 33, 12001, "rowstream", False)])
+def test_summed_splits_match_the_reduce_launch(m, n, k, kernel, summed):
+    import hc.gfx950 as g
     from hc.gfx950 import _native
 
     print(f"case summed splits m={m} n={n} k={k}", flush=True)
@@ -180,6 +198,9 @@ def test_summed_splits_match_the_reduce_launch(m, n, k):
             outs.append(c)
         torch.cuda.synchronize()
         assert torch.equal(outs[0], outs[1]), rnd
+    names = _kernels_of(lambda: g.gemm(a, b, out=outs[0]))
+    assert any(f"gemm_{kernel}_kernel" in name for name in names), names
+    assert any("reduce" in name for name in names) == (not summed), names
 
 
 # 17 to 64 rows and 33 to 64 columns: small operands take the tiled kernel,
@@ -215,18 +236,6 @@ def test_few_rows_or_columns_of_a_wide_matrix_stream(m, n, k, lda, ldb, algo):
     want = a.double() @ b.double()
     # 32-bit sums of k exact products, in any order: each within k units of 2^-24 of the sum of magnitudes.
     assert ((got - want).abs() <= k * 2.0**-24 * (a.double().abs() @ b.double().abs())).all()
-
-
-def _kernels_of(fn):
-    """Names of the kernels a call runs."""
-    from torch.profiler import ProfilerActivity, profile
-
-    fn()
-    torch.cuda.synchronize()
-    with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as prof:
-        fn()
-        torch.cuda.synchronize()
-    return [e.name for e in prof.events() if e.device_type == torch.autograd.DeviceType.CUDA]
 
 
 # Rows so far apart that an operand spans 2 GiB: the WIDE form of
