@@ -3386,7 +3386,10 @@ int gemm_impl(int algo, int dtype, const void* A, int64_t lda, const void* B, in
   // 64 x 1000 x 1000 8.5 -> 6.1, 64 x 8192 x 4096 (64 MiB) 17.7 -> 15.3, 64 x 8192 x 8192 30.4 / 32.1;
   // 2048 x 33 x 512 6.3 -> 4.8, 4096 x 64 x 8192 17.9 -> 14.0, 8192 x 64 x 8192
   // 31.9 / 33.4.  With 17 to 32 columns they are even (4000 x 17 x 2000 8.6 /
-  // 9.2), and 16 rows (16 x 4000 x 2000 8.2 / 8.9) or fewer stream.  Rows
+  // 9.2), and 16 rows (16 x 4000 x 2000 8.2 / 8.9) or fewer stream.  Past one
+  // 64-column tile per CU a short K streams too: 17 x 17000 x 300 5.1 / 5.8,
+  // 24 x 32000 x 128 4.3 / 4.8, 17 x 20000 x 512 6.3 / 6.5, 17 x 20000 x 800
+  // 8.3 / 8.1, 48 x 20000 x 64 4.1 / 4.7, 48 x 17000 x 200 5.4 / 5.1.  Rows
   // 65 .. 128 go to the tiled kernel whatever B's size.  It needs the large
   // operand readable in place, and both within 32-bit offsets as they are
   // strided: past those there are no small tiles and no K split, only
@@ -3398,6 +3401,7 @@ int gemm_impl(int algo, int dtype, const void* A, int64_t lda, const void* B, in
     return (whole && aligned16(p) && ld % 8 == 0) || (aligned2(p) && chunk_tail_readable(p, rows, cols, ld));
   };
   const bool mid = algo == HCG_ALGO_AUTO && M > 16 && N > 32 && K <= (M > 32 ? 8192 : 4096) &&
+                   (N <= 64 * (int64_t)st->num_cus || (M > 32 ? K > 128 : 32 * K > N)) &&
                    fast_extents_fit((int)M, (int)N, (int)K, lda, ldb);
   const bool tiled_cols = mid && N <= 64 && 2 * M * K <= kCached && in_place(A, M, K, lda, K % 8 == 0);
   const bool use_narrow = algo == HCG_ALGO_NARROW ||

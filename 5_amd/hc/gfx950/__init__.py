@@ -202,8 +202,8 @@ def gemm(a: Any, b: Any, out: Any | None = None, *, algo: str = "auto", device: 
 
     ``algo``: "auto" (the library picks: streaming kernels for N <= 64 and
     for M <= 64, except that 33 columns or 17 rows and more of at most
-    64 MiB and a K of at most 8192 (strided over less than 2 GiB) take the
-    LDS-tiled kernel, and for
+    64 MiB and a K of at most 8192 (strided over less than 2 GiB, and not
+    too short past 16384 columns) take the LDS-tiled kernel, and for
     M <= 128 when the tiled kernel cannot read B in place; otherwise the
     LDS-tiled kernel with a modelled tile shape and K split, with up to 128
     rows or 64 columns past a multiple of 256 peeled off to a streaming

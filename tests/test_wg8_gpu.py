@@ -323,3 +323,21 @@ def test_transposed_b_under_many_rows_is_copied(m, n, k, copied):
     assert torch.isnan(c).all() if copied else torch.equal(c, want)
     at = a[:8200].t().contiguous().t()
     assert torch.equal(g.gemm(at, bt.t().contiguous()), want[:8200])
+
+
+# Past one 64-column tile per CU, 17 to 32 rows with K up to N / 32 and 33 to 64
+# with K up to 128 stream.
+@pytest.mark.parametrize("m,n,k,kernel", [(17, 16384, 96, "wg8"), (17, 16385, 96, "stream"), (32, 16640, 520, "stream"),
+                                          (32, 16640, 521, "wg8"), (33, 16400, 128, "stream"),
+                                          (64, 16400, 129, "wg8")])
+def test_short_k_past_one_tile_per_cu_streams(m, n, k, kernel):
+    import hc.gfx950 as g
+
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the line is one 64-column tile per CU, stated here for 256")
+    _check(m, n, k, "float16", 8)
+    a = torch.zeros(m, k, dtype=torch.float16, device=DEV)
+    b = torch.zeros(k, n, dtype=torch.float16, device=DEV)
+    out = torch.empty(m, n, device=DEV)
+    names = _kernels_of(lambda: g.gemm(a, b, out=out))
+    assert any(f"gemm_{kernel}_kernel" in name for name in names), names
