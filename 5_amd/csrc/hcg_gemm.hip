@@ -2498,7 +2498,9 @@ constexpr double kLaunchUs = 2.0;
 // of the parts, bit-reproducibly: by the tile's last workgroup to arrive
 // (fused: wg8 tiles of at most 128x128), or by a second launch.  Fused, the
 // tail of a workgroup grows by 1 us (write-through, atomic) plus the other
-// partials' loads at 100 KB/us by one CU, plus the partials' traffic; the
+// partials' loads at 100 KB/us by one CU, at least 0.23 us each (priced by
+// their 16 KB alone, 64x64 tiles were split too far: 32 x 1000 x 3584 8 parts 8.2,
+// 6 parts 7.5; 600 x 40 x 8192 12 parts 9.4, 8 parts 8.4), plus the partials' traffic; the
 // second launch costs 3 to 6 us (boxes differ by the gap between launches)
 // plus the traffic, and 2.5 us of host time, so that small calls take at
 // least 6.6 us.  Both sides, us: 128 x 8192 x 8192 (4 parts of 64 KB) 34.4
@@ -2549,7 +2551,7 @@ double plan_cost(const TileShape& t, int splits, bool fused, int num_cus, int M,
   double us = kLaunchUs + (double)rounds * t.fixed + (double)(per_cu * nk) * (t.lo + (t.hi - t.lo) * busy);
   if (splits > 1) {
     if (fused) {
-      us += 1.0 + (splits - 1) * (t.tm * t.tn * 4) / 1.0e5 + (double)fused_bytes(t, splits, M, N) / 3.0e6;
+      us += 1.0 + (splits - 1) * fmax(0.234, (t.tm * t.tn * 4) / 1.0e5) + (double)fused_bytes(t, splits, M, N) / 3.0e6;
     } else {
       us += 5.0 + (double)(splits + 1) * M * N * sizeof(float) / 4.5e6;
       if (us < 6.6) us = 6.6;
