@@ -143,17 +143,6 @@ def test_transposed_operand_under_capture():
         assert torch.equal(out, eager)
 
 
-# Over 1.25 row blocks of 64 per CU the narrow kernel walks several blocks per
-# workgroup: a block's last stage beside the next one's first, K of one stage
-# (so that every stage ends a block), below one and ragged, the last block
-# ragged, workgroups with one block more than others.
-@pytest.mark.parametrize("m,n,k", [(20481, 8, 128), (20417, 1, 1), (33000, 16, 130), (40963, 17, 500), (24000, 33, 1001),
-                                   (32768, 64, 640), (50001, 40, 257)])
-@pytest.mark.parametrize("dtype", list(DTYPES))
-def test_narrow_kernel_walks_row_blocks(m, n, k, dtype):
-    _check(m, n, k, dtype, 3 if dtype == "float16" else 8)
-
-
 def _kernels_of(fn):
     """Names of the kernels a call runs."""
     from torch.profiler import ProfilerActivity, profile
@@ -164,6 +153,32 @@ def _kernels_of(fn):
         fn()
         torch.cuda.synchronize()
     return [e.name for e in prof.events() if e.device_type == torch.autograd.DeviceType.CUDA]
+
+
+# Over 1.25 row blocks of 64 per CU the narrow kernel walks several blocks per
+# workgroup: a block's last stage beside the next one's first, K of one stage
+# (so that every stage ends a block), below one and ragged, the last block
+# ragged, workgroups with one block more than others.  33 to 64 columns of at
+# most 64 MiB go to the tiled kernel unless the narrow one is asked for.
+@pytest.mark.parametrize("m,n,k,algo", [(20481, 8, 128, "auto"), (20417, 1, 1, "auto"), (33000, 16, 130, "auto"),
+                                        (40963, 17, 500, "auto"), (24000, 33, 1001, "narrow"),
+                                        (32768, 64, 640, "narrow"), (50001, 40, 257, "narrow"),
+                                        (20417, 50, 64, "narrow"), (40001, 40, 1001, "auto"),
+                                        (20500, 64, 4096, "auto")])
+@pytest.mark.parametrize("dtype", list(DTYPES))
+def test_narrow_kernel_walks_row_blocks(m, n, k, algo, dtype):
+    import hc.gfx950 as g
+
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the line is 1.25 row blocks per CU, stated here for 256")
+    _check(m, n, k, dtype, 3 if dtype == "float16" else 8, algo)
+    a = torch.zeros(m, k, dtype=DTYPES[dtype], device=DEV)
+    b = torch.zeros(k, n, dtype=DTYPES[dtype], device=DEV)
+    out = torch.empty(m, n, device=DEV)
+    names = _kernels_of(lambda: g.gemm(a, b, out=out, algo=algo))
+    block = 16 if n <= 16 else 32 if n <= 32 else 64
+    walking = f"gemm_rowstream_kernel<{list(DTYPES).index(dtype)}, {block}, false, 0, true>"
+    assert any(walking in name for name in names), names
 
 
 # K splits summed by a block's last workgroup against the same partials summed
