@@ -241,7 +241,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wg8_kernel(Args g) {
   static_assert(MI >= 1 && NI >= 1, "wave tile");
   constexpr int KW = KS / WK;     // k per wave per stage
   constexpr int NSUB = KW / 16;   // 16-wide K steps per wave per stage
-  static_assert(NSUB == 2 || NSUB == 4 || NSUB == 1, "K steps");
+  static_assert(NSUB == 2 || NSUB == 4, "K steps");
+  static_assert(STAGES == 3 || STAGES == 4, "stages");
   using OpA = Operand<TM, KS, AKC>;
   using OpB = Operand<TN, KS, BKC>;
   constexpr int kStageBytes = OpA::kBytes + OpB::kBytes;
@@ -363,30 +364,13 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wg8_kernel(Args g) {
       else
         schedule(std::integral_constant<int, 0>{});
     }
-    if constexpr (kPre == 0) issue_b(StageC<(S + STAGES - 1) % STAGES>{}, full, kt + STAGES - 1);
     wait_vm<(STAGES - 2) * kDma>();
     wait_lgkm();
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (NSUB == 1) {
-      // One K step per stage: its fragments live in set 0 only, so the next
-      // stage's go to set 1 and are moved after the multiply.
-      u32x4 ka[MI], kb[NI];
-#pragma unroll
-      for (int i = 0; i < MI; ++i) ka[i] = fa[0][i];
-#pragma unroll
-      for (int j = 0; j < NI; ++j) kb[j] = fb[0][j];
-      read(StageC<(S + 1) % STAGES>{}, 0, Mask{}, kt + 1);
-      issue_a(sc, full, kt + STAGES);
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NI; ++j) acc[i][j] = mfma<DT>(ka[i], kb[j], acc[i][j]);
-    } else {
-      read(StageC<(S + 1) % STAGES>{}, 0, Mask{}, kt + 1);
-      issue_a(sc, full, kt + STAGES);
-      multiply(NSUB - 1);
-    }
+    read(StageC<(S + 1) % STAGES>{}, 0, Mask{}, kt + 1);
+    issue_a(sc, full, kt + STAGES);
+    multiply(NSUB - 1);
     schedule(std::integral_constant<int, OpA::kInst>{});
   };
 
@@ -394,17 +378,11 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wg8_kernel(Args g) {
   using Checked = std::false_type;
   issue_a(StageC<0>{}, Checked{}, 0);
   issue_b(StageC<0>{}, Checked{}, 0);
-  if constexpr (STAGES > 2) {
-    issue_a(StageC<1>{}, Checked{}, 1);
-    issue_b(StageC<1>{}, Checked{}, 1);
-  }
+  issue_a(StageC<1>{}, Checked{}, 1);
+  issue_b(StageC<1>{}, Checked{}, 1);
   if constexpr (STAGES > 3) {
     issue_a(StageC<2>{}, Checked{}, 2);
     issue_b(StageC<2>{}, Checked{}, 2);
-  }
-  if constexpr (STAGES > 4) {
-    issue_a(StageC<3>{}, Checked{}, 3);
-    issue_b(StageC<3>{}, Checked{}, 3);
   }
   issue_a(StageC<STAGES - 1>{}, Checked{}, STAGES - 1);
   wait_vm<(STAGES - 2) * kDma + OpA::kInst>();
@@ -417,25 +395,20 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_wg8_kernel(Args g) {
   const int nfull = g.K / KS;
   for (; kt + 2 * STAGES <= nfull; kt += STAGES) {
     iteration(StageC<0>{}, Full{}, kt);
-    iteration(StageC<1 % STAGES>{}, Full{}, kt + 1);
-    if constexpr (STAGES > 2) iteration(StageC<2 % STAGES>{}, Full{}, kt + 2);
+    iteration(StageC<1>{}, Full{}, kt + 1);
+    iteration(StageC<2>{}, Full{}, kt + 2);
     if constexpr (STAGES > 3) iteration(StageC<3 % STAGES>{}, Full{}, kt + 3);
-    if constexpr (STAGES > 4) iteration(StageC<4 % STAGES>{}, Full{}, kt + 4);
   }
   for (; kt + STAGES <= nk; kt += STAGES) {
     iteration(StageC<0>{}, Checked{}, kt);
-    iteration(StageC<1 % STAGES>{}, Checked{}, kt + 1);
-    if constexpr (STAGES > 2) iteration(StageC<2 % STAGES>{}, Checked{}, kt + 2);
+    iteration(StageC<1>{}, Checked{}, kt + 1);
+    iteration(StageC<2>{}, Checked{}, kt + 2);
     if constexpr (STAGES > 3) iteration(StageC<3 % STAGES>{}, Checked{}, kt + 3);
-    if constexpr (STAGES > 4) iteration(StageC<4 % STAGES>{}, Checked{}, kt + 4);
   }
   if (kt < nk) iteration(StageC<0>{}, Checked{}, kt++);
-  if constexpr (STAGES > 2)
-    if (kt < nk) iteration(StageC<1 % STAGES>{}, Checked{}, kt++);
+  if (kt < nk) iteration(StageC<1>{}, Checked{}, kt++);
   if constexpr (STAGES > 3)
-    if (kt < nk) iteration(StageC<2 % STAGES>{}, Checked{}, kt++);
-  if constexpr (STAGES > 4)
-    if (kt < nk) iteration(StageC<3 % STAGES>{}, Checked{}, kt++);
+    if (kt < nk) iteration(StageC<2>{}, Checked{}, kt++);
   wait_vm<0>();  // no DMA may still be writing LDS
   stamps.mark(2);
   __builtin_amdgcn_s_barrier();  // every wave is done reading the stages
