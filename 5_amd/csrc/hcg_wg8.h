@@ -14,15 +14,14 @@
 // of the 239 bytes per cycle that eight reach, and 64x64 of accumulators per
 // wave need 128 per cycle of MFMA issue.  Eight waves (two per SIMD) and 96
 // KB in flight per CU took 2048^3 bf16 from 23.9 to 18.8 us; per-workgroup
-// timestamps: K loop 12.8 us, 670 cycles per 64-wide step against 512 of MFMA
-// issue, at 1670 MHz (the board's power limit; the same loop of 128x256 tiles
-// on 4096 x 2048 x 2048 issues MFMAs in 94% of its cycles, at 1410 MHz),
-// prologue 1.7, epilogue 2.0 (16 MiB of C).  Two K groups (WK = 2) keep the
-// wave tile square at 64x64 where the workgroup's is 128x128: 64 KB of LDS
-// reads per 64-wide step, against 96 KB for eight 64x32 wave tiles.  Small
-// tiles are bound by the DMA (64 bytes per cycle per CU): 64x64 takes 380
-// cycles per step, 256 of them DMA and 128 MFMA, and wins by filling CUs:
-// 1024^3 12.3 -> 6.5 us, 512^3 6.7 -> 4.2.
+// timestamps: K loop 12.0 us (14.0 on a slower board), 693 (670) cycles per
+// 64-wide step against 512 of MFMA issue, at 1.95 (1.69) GHz, prologue 1.7,
+// epilogue 2.0 (16 MiB of C); 128x256 tiles on 4096 x 2048 x 2048 24.8 us, 1380
+// cycles against 1024.  Two K groups (WK = 2) keep the wave tile square at 64x64
+// where the workgroup's is 128x128: 64 KB of LDS reads per 64-wide step, against
+// 96 KB for eight 64x32 wave tiles.  Small tiles are bound by the DMA (64 bytes
+// per cycle per CU): 64x64 takes 344 to 396 cycles per step, 256 of them DMA and
+// 128 MFMA, and wins by filling CUs: 1024^3 12.3 -> 6.5 us, 512^3 6.7 -> 4.2.
 #pragma once
 
 #include <hip/hip_runtime.h>
