@@ -356,3 +356,20 @@ def test_short_k_past_one_tile_per_cu_streams(m, n, k, kernel):
     out = torch.empty(m, n, device=DEV)
     names = _kernels_of(lambda: g.gemm(a, b, out=out))
     assert any(f"gemm_{kernel}_kernel" in name for name in names), names
+
+
+# A remainder past a multiple of 256 is peeled onto a streaming kernel only for
+# a gain the model can tell.
+@pytest.mark.parametrize("m,n,k,peeled", [(4209, 3984, 552, False), (5440, 2848, 513, False), (4100, 4096, 768, True)])
+def test_remainders_are_peeled_for_a_clear_gain(m, n, k, peeled):
+    import hc.gfx950 as g
+
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the model's gains are stated here for 256 CUs")
+    _check(m, n, k, "float16", 8)
+    a = torch.zeros(m, k, dtype=torch.float16, device=DEV)
+    b = torch.zeros(k, n, dtype=torch.float16, device=DEV)
+    out = torch.empty(m, n, device=DEV)
+    names = _kernels_of(lambda: g.gemm(a, b, out=out))
+    assert any("gemm_dma_kernel" in name for name in names)
+    assert any("gemm_stream_kernel" in name or "gemm_rowstream_kernel" in name for name in names) == peeled, names
